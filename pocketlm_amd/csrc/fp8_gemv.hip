@@ -35,6 +35,8 @@
 #include <vector>
 
 #include "common.h"
+#include "fp8_batch.h"
+#include "fp8_mfma.h"
 #include "route.h"
 
 // Loads of down-phase items (or lanes) that do not count read these zero
@@ -45,6 +47,8 @@
 static __device__ __align__(256) unsigned char down_zero_page[256];
 
 namespace {
+
+using namespace plm_fp8;
 
 constexpr int kMaxGroups = 64;  // experts per launch (pointer tables travel as kernel arguments)
 constexpr int kMaxWaves = 8;
@@ -429,122 +433,8 @@ __global__ __launch_bounds__(512) void moe_route_plan_kernel(const float* __rest
 // the value, lo = 0).  Rows and activations without such values give the
 // same bits in both passes.
 
-typedef __bf16 plm_bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 plm_bf16x2 __attribute__((ext_vector_type(2)));
-typedef float plm_f32x4 __attribute__((ext_vector_type(4)));
-
-// Weight bytes are read once per call: nontemporal loads keep them from
-// displacing the activations and scales in the caches.
-__device__ __forceinline__ plm_u32x4 wload16(const void* p) {
-    return __builtin_nontemporal_load((const __attribute__((address_space(1))) plm_u32x4*)(p));
-}
-
-__device__ __forceinline__ plm_u32x4 xload16(const void* p) {
-    return *(const __attribute__((address_space(1))) plm_u32x4*)(p);
-}
-
-template <bool HI>
-__device__ __forceinline__ uint32_t e4m3_pair_to_bf16(uint32_t v) {
-    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 1.0f, HI));
-}
-
-// 16 e4m3 bytes -> the two A operands (bytes 0-7, 8-15)
-__device__ __forceinline__ void weights_to_bf16(const plm_u32x4 q, plm_bf16x8& a0, plm_bf16x8& a1) {
-    const plm_u32x4 t0 = {e4m3_pair_to_bf16<false>(q.x), e4m3_pair_to_bf16<true>(q.x),
-                          e4m3_pair_to_bf16<false>(q.y), e4m3_pair_to_bf16<true>(q.y)};
-    const plm_u32x4 t1 = {e4m3_pair_to_bf16<false>(q.z), e4m3_pair_to_bf16<true>(q.z),
-                          e4m3_pair_to_bf16<false>(q.w), e4m3_pair_to_bf16<true>(q.w)};
-    a0 = __builtin_bit_cast(plm_bf16x8, t0);
-    a1 = __builtin_bit_cast(plm_bf16x8, t1);
-}
-
-// NaN bytes (0x7F, 0xFF) -> 0
-__device__ __forceinline__ plm_u32x4 zero_nan_bytes(plm_u32x4 q) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const uint32_t w = q[k];
-        const uint32_t nan = ((w & 0x7F7F7F7Fu) + 0x01010101u) & 0x80808080u;  // 0x80 where the low 7 bits are all 1
-        q[k] = w & ~((nan >> 7) * 0xFFu);
-    }
-    return q;
-}
-
-// hi / lo bf16 halves of one fp32 value.  EXACT: infinities and NaNs go to hi
-// whole (a quiet NaN for every NaN) with lo = 0.
-template <bool EXACT>
-__device__ __forceinline__ void split_f32(uint32_t x, uint32_t& hi, uint32_t& lo) {
-    hi = x >> 16;
-    const float rem = __uint_as_float(x) - __uint_as_float(x & 0xFFFF0000u);
-    lo = __builtin_bit_cast(uint16_t, static_cast<__bf16>(rem));
-    if constexpr (EXACT) {
-        if ((x & 0x7F800000u) == 0x7F800000u) {
-            hi = (x & 0x007FFFFFu) != 0 ? 0x7FC0u : hi;
-            lo = 0;
-        }
-    }
-}
-
-// 8 fp32 activations (two loads) -> hi and lo B operands
-template <bool EXACT>
-__device__ __forceinline__ void split8(const plm_u32x4 v0, const plm_u32x4 v1, plm_bf16x8& hi, plm_bf16x8& lo) {
-    const uint32_t x[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-    plm_u32x4 h, l;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        if constexpr (EXACT) {
-            uint32_t h0, l0, h1, l1;
-            split_f32<true>(x[2 * p], h0, l0);
-            split_f32<true>(x[2 * p + 1], h1, l1);
-            h[p] = h0 | (h1 << 16);
-            l[p] = l0 | (l1 << 16);
-        } else {
-            h[p] = __builtin_amdgcn_perm(x[2 * p + 1], x[2 * p], 0x07060302u);
-            const float r0 = __uint_as_float(x[2 * p]) - __uint_as_float(x[2 * p] & 0xFFFF0000u);
-            const float r1 = __uint_as_float(x[2 * p + 1]) - __uint_as_float(x[2 * p + 1] & 0xFFFF0000u);
-            const plm_float2 rr = {r0, r1};
-            l[p] = __builtin_bit_cast(uint32_t, __builtin_convertvector(rr, plm_bf16x2));
-        }
-    }
-    hi = __builtin_bit_cast(plm_bf16x8, h);
-    lo = __builtin_bit_cast(plm_bf16x8, l);
-}
-
-__device__ __forceinline__ plm_f32x4 mfma_bf16(plm_bf16x8 a, plm_bf16x8 b, plm_f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-// The activations of one block for the lane's B column: two bf16 loads, or
-// four fp32 loads (split into hi and lo later).
-template <bool XB>
-struct XPiece {
-    plm_u32x4 v[XB ? 2 : 4];
-};
-
-template <bool XB>
-__device__ __forceinline__ XPiece<XB> load_xpiece(const void* p, bool live) {
-    XPiece<XB> r;
-    const char* c = static_cast<const char*>(p);
-#pragma unroll
-    for (int k = 0; k < (XB ? 2 : 4); ++k) r.v[k] = live ? xload16(c + 16 * k) : plm_u32x4{0, 0, 0, 0};
-    return r;
-}
-
 // D of one tile and block: the A operands from the weights q against the
 // activation piece x.
-template <bool XB, bool SAN>
-struct BOperands {
-    plm_bf16x8 h0, h1, l0, l1;
-    __device__ __forceinline__ explicit BOperands(const XPiece<XB>& x) {
-        if constexpr (XB) {
-            h0 = __builtin_bit_cast(plm_bf16x8, x.v[0]);
-            h1 = __builtin_bit_cast(plm_bf16x8, x.v[1]);
-        } else {
-            split8<SAN>(x.v[0], x.v[1], h0, l0);
-            split8<SAN>(x.v[2], x.v[3], h1, l1);
-        }
-    }
-};
-
 template <bool XB, bool SAN>
 __device__ __forceinline__ plm_f32x4 tile_block(plm_u32x4 q, const BOperands<XB, SAN>& b) {
     plm_bf16x8 a0, a1;
@@ -579,44 +469,6 @@ __device__ __forceinline__ void halves_to_lds(const plm_f32x4 (&acc)[NT], float*
             const float v = acc[t][j] + __shfl(acc[t][j], (lane + 40) & 63);
             if (lane < 24 && (lane & 15) < 8) red[(slot * NT + t) * 64 + (4 * (lane >> 4) + j) * 8 + (lane & 7)] = v;
         }
-}
-
-// The SiLU intermediate silu(gate) * up as the down phase reads it: bf16
-// hi / lo planes (exact for infinities and NaNs).
-__device__ __forceinline__ void store_hplanes(uint16_t* hi, uint16_t* lo, int64_t o, float v) {
-    uint32_t h, l;
-    split_f32<true>(__float_as_uint(v), h, l);
-    hi[o] = static_cast<uint16_t>(h);
-    lo[o] = static_cast<uint16_t>(l);
-}
-
-__device__ __forceinline__ float lane_value(float v, int k) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), k));
-}
-
-// Runs nk steps through P register slots, pipelined: P steps are in
-// flight and step k + P is issued into the slot step k leaves; the steps
-// beyond a multiple of P run first, unpipelined.
-template <int P, class Issue, class Compute>
-__device__ __forceinline__ void run_pipelined(int nk, Issue& issue, Compute& compute) {
-    const int r = nk % P;
-    for (int k = 0; k < r; ++k) {
-        issue(0, k);
-        compute(0, k);
-    }
-    if (nk > r) {
-#pragma unroll
-        for (int u = 0; u < P; ++u) issue(u, r + u);
-        for (int k0 = r; k0 + P < nk; k0 += P) {
-#pragma unroll
-            for (int u = 0; u < P; ++u) {
-                compute(u, k0 + u);
-                issue(u, k0 + u + P);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < P; ++u) compute(u, nk - P + u);
-    }
 }
 
 // The burst schedule of a rows-kernel wave (the MoE's gate/up launches):
@@ -1889,12 +1741,50 @@ bool rows_fast_ok(const RowsProblem& p) {
     return true;
 }
 
+// More than kMaxM activation rows on the vector path: whole MFMA tiles
+// (fp8_batch.hip), one launch per weight set; the same bits per row.
+int run_rows_batch(const RowsProblem& p, hipStream_t st) {
+    const int outs = p.silu ? 1 : p.nwt;  // gate and up share a launch
+    for (int i = 0; i < outs; ++i)
+        for (int g0 = 0; g0 < p.ngroups; g0 += p.nvar > 0 ? 1 : kMaxGroups) {
+            plm::BatchRows b;
+            b.ngroups = p.nvar > 0 ? 1 : std::min(kMaxGroups, p.ngroups - g0);
+            for (int g = 0; g < b.ngroups; ++g)
+                for (int k = 0; k < (p.silu ? 2 : 1); ++k) {
+                    b.w[k][g] = p.w[i + k][g0 + g];
+                    b.s[k][g] = p.s[i + k][g0 + g];
+                }
+            b.x = p.x;
+            b.xb = p.xb;
+            b.x_stride = p.x_stride;
+            b.rows = p.nvar > 0 ? p.vrows[g0] : p.rows;
+            b.K = p.K;
+            b.scale_cols = p.scale_cols;
+            b.m = p.batch;
+            const int64_t nb = plm::ceil_div(p.K, 128);
+            b.waves = p.silu ? rows_waves<true>(nb) : rows_waves<false>(nb);
+            b.tiled = p.tiled;
+            const int64_t goff = static_cast<int64_t>(g0) * p.batch * p.out_ld;
+            if (p.silu) {
+                uint16_t* planes = reinterpret_cast<uint16_t*>(p.out[0]);
+                b.hhi = planes + goff;
+                b.hlo = planes + static_cast<int64_t>(p.ngroups) * p.batch * p.out_ld + goff;
+            } else {
+                b.out = p.nvar > 0 ? p.vout[g0] : p.out[i] + goff;
+            }
+            const int code = plm::fp8_batch_rows(b, st);
+            if (code != 0) return code;
+        }
+    return 0;
+}
+
 int run_rows(const RowsProblem& p, hipStream_t st) {
     const bool fast = rows_fast_ok(p);
     if (p.tiled && (!fast || p.nvar > 0))
         return plm::fail(-2, "8-row tile weights need K %% 16 == 0 and 16-byte aligned weights and activations");
     if (p.nvar > 0 && (!fast || p.nwt != 1 || p.ngroups != p.nvar || p.nvar > kMaxVar))
         return plm::fail(-2, "variable-row groups need the vector path and one weight per group");
+    if (fast && p.batch > kMaxM) return run_rows_batch(p, st);
     for (int g0 = 0; g0 < p.ngroups; g0 += kMaxGroups) {
         const int ng = std::min(kMaxGroups, p.ngroups - g0);
         RowsArgs a;
@@ -1980,11 +1870,42 @@ struct CombineProblem {
     int64_t scale_cols;
 };
 
+// More than kMaxM activation rows of unweighted groups with outputs of their
+// own (the MLP, the many-expert MLP): fp8_batch.hip, the same bits per row.
+int run_combine_batch(const CombineProblem& p, hipStream_t st) {
+    const uint16_t* hi = reinterpret_cast<const uint16_t*>(p.act);
+    const uint16_t* lo = hi + static_cast<int64_t>(p.ngroups) * p.batch * p.K;
+    for (int g0 = 0; g0 < p.ngroups; g0 += kMaxGroups) {
+        plm::BatchRows b;
+        b.ngroups = std::min(kMaxGroups, p.ngroups - g0);
+        for (int g = 0; g < b.ngroups; ++g) {
+            b.w[0][g] = p.w[g0 + g];
+            b.s[0][g] = p.s[g0 + g];
+        }
+        const int64_t row0 = static_cast<int64_t>(g0) * p.batch;
+        b.xhi = hi + row0 * p.K;
+        b.xlo = lo + row0 * p.K;
+        b.x_stride = p.K;
+        b.out = p.out + row0 * p.rows;
+        b.rows = p.rows;
+        b.K = p.K;
+        b.scale_cols = p.scale_cols;
+        b.m = p.batch;
+        b.waves = static_cast<int>(std::min<int64_t>(plm::ceil_div(p.K, 128), plm::kBatchDownWaves));
+        const int code = plm::fp8_batch_rows(b, st);
+        if (code != 0) return code;
+    }
+    return 0;
+}
+
 int run_combine(const CombineProblem& p, hipStream_t st) {
     if (p.out_last != nullptr && (p.per_group_out || p.ngroups < 2 || p.ngroups > kMaxGroups))
         return plm::fail(-2, "a split-off last group needs 2..%d summed groups", kMaxGroups);
     bool fast = p.K % 16 == 0 && plm::aligned16(p.act);
     for (int g = 0; g < p.ngroups && fast; ++g) fast = plm::aligned16(p.w[g]);
+    if (fast && p.batch > kMaxM && p.route == nullptr && p.out_last == nullptr &&
+        (p.per_group_out || p.ngroups == 1))
+        return run_combine_batch(p, st);
     for (int g0 = 0; g0 < p.ngroups; g0 += kMaxGroups) {
         const int ng = std::min(kMaxGroups, p.ngroups - g0);
         CombineArgs a;
@@ -2276,6 +2197,39 @@ int pair_weighted_impl(const uint64_t* gp, const uint64_t* gsp, const uint64_t* 
         for (int64_t p = 0; p < pair_count; ++p) {
             if (items[p] < 0 || items[p] >= expert_count || rows[p] < 0 || rows[p] >= batch)
                 return plm::fail(-4, "pair %lld out of range", static_cast<long long>(p));
+        }
+    }
+    // A prompt chunk: each expert on the rows that chose it.
+    if (batch > kMaxM && inter % 16 == 0 && hid % 16 == 0 &&
+        plm::aligned16(hidden.f32 != nullptr ? static_cast<const void*>(hidden.f32) : hidden.bf16)) {
+        ExpertTables t(gp, gsp, up, usp, dp, dsp, expert_count);
+        bool vec = true;
+        for (int64_t e = 0; e < expert_count && vec; ++e)
+            vec = plm::aligned16(t.g[e]) && plm::aligned16(t.u[e]) && plm::aligned16(t.d[e]);
+        if (vec) {
+            plm::PairProblem p;
+            p.w[0] = t.g.data();
+            p.w[1] = t.u.data();
+            p.w[2] = t.d.data();
+            p.s[0] = t.gs.data();
+            p.s[1] = t.us.data();
+            p.s[2] = t.ds.data();
+            p.x = hidden.f32;
+            p.xb = hidden.bf16;
+            p.items = pair_item_indices;
+            p.rows = pair_row_indices;
+            p.weights = pair_weights;
+            p.out = out;
+            p.bad = bad_pairs;
+            p.experts = expert_count;
+            p.pairs = pair_count;
+            p.batch = batch;
+            p.inter = inter;
+            p.hid = hid;
+            p.gsc = gsc;
+            p.dsc = dsc;
+            p.gate_waves = rows_waves<true>(plm::ceil_div(hid, 128));
+            return plm::fp8_batch_pairs(p, st);
         }
     }
     // Dense route matrix [E, batch] after the activations in the workspace.

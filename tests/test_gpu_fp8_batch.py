@@ -1,0 +1,111 @@
+"""FP8 projections of nine or more activation rows (whole MFMA tiles) and the
+routed experts on the (expert, row) pairs of a prompt chunk, at sizes on the
+edges of the row, column and token tiles.
+
+Bars: linear, dual and MLP rows have the bits of one-row calls.  The pairs
+are held to the oracle, whose sums run in another order: fp32 sums, fp32
+activations and the SiLU intermediate as bf16 hi + lo (at most 2^-17 relative
+each), rel-L2 2e-5.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def nat():
+    from pocketlm_amd import native
+
+    assert native.native_fp8_linear_available(), "libpocketlm_hip.so must load on the GPU box"
+    return native
+
+
+def _fp8(rows, cols, seed, nan_at=()):
+    g = torch.Generator().manual_seed(seed)
+    w = (torch.randn((rows, cols), generator=g) * 0.02).to(torch.float8_e4m3fn).view(torch.uint8)
+    for r, c in nan_at:
+        w[r, c] = 0x7F
+    s = torch.rand(((rows + 127) // 128, (cols + 127) // 128), generator=g) * 9e-3 + 1e-3
+    return w.cuda(), s.cuda()
+
+
+def _x(m, k, seed, dtype):
+    return torch.randn((m, k), generator=torch.Generator().manual_seed(seed)).to(dtype).cuda()
+
+
+def _rows_of(fn, x, at):
+    return torch.cat([fn(x[i:i + 1]) for i in at])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,cols", [(72, 144), (200, 2064), (576, 7168), (130, 1024)])
+def test_rows_have_the_bits_of_one_row_calls(nat, rows, cols, dtype):
+    w, s = _fp8(rows, cols, rows + cols, nan_at=[(rows - 1, 17)])
+    w2, s2 = _fp8(rows, cols, rows + cols + 1)
+    for m in (9, 16, 17, 33, 64, 65, 129, 150):
+        print("linear", rows, cols, m, dtype, flush=True)
+        x = _x(m, cols, m, dtype)
+        at = sorted({0, 8, 15, 16, m // 2, m - 2, m - 1} & set(range(m)))
+        y = nat.fp8_e4m3_block_linear_f32(w, s, x)
+        assert torch.isfinite(y).all()
+        assert torch.equal(y[at], _rows_of(lambda r: nat.fp8_e4m3_block_linear_f32(w, s, r), x, at)), m
+        ya, yb = nat.fp8_e4m3_block_dual_linear_f32(w, s, w2, s2, x)
+        assert torch.equal(ya, y) and torch.equal(yb, nat.fp8_e4m3_block_linear_f32(w2, s2, x)), m
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("inter,hid", [(144, 400), (272, 1040), (2048, 512)])
+def test_mlp_rows_have_the_bits_of_one_row_calls(nat, inter, hid, dtype):
+    args = [*_fp8(inter, hid, 1, nan_at=[(3, 5)]), *_fp8(inter, hid, 2), *_fp8(hid, inter, 3, nan_at=[(hid - 1, 0)])]
+    for m in (9, 16, 31, 65, 129, 150):
+        print("mlp", inter, hid, m, dtype, flush=True)
+        x = _x(m, hid, m, dtype)
+        at = sorted({0, 8, 15, 16, m // 2, m - 1} & set(range(m)))
+        y = nat.fp8_e4m3_block_mlp_f32(*args, x)
+        assert torch.equal(y[at], _rows_of(lambda r: nat.fp8_e4m3_block_mlp_f32(*args, r), x, at)), m
+
+
+def test_infinite_activation_among_many_rows(nat):
+    w, s = _fp8(192, 512, 77)
+    x = _x(20, 512, 78, torch.float32)
+    x[3, 130] = float("inf")
+    x[17, 5] = -float("inf")
+    y = nat.fp8_e4m3_block_linear_f32(w, s, x)
+    want = _rows_of(lambda r: nat.fp8_e4m3_block_linear_f32(w, s, r), x, range(20))
+    assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y.nan_to_num(), want.nan_to_num())
+    assert y[3].isinf().any() and torch.isfinite(y[4]).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("experts,batch,inter,hid,top", [(3, 9, 144, 400, 1), (70, 40, 128, 272, 4),
+                                                         (2, 33, 272, 528, 2), (5, 300, 128, 128, 2)])
+def test_pairs_vs_the_oracle(nat, oracle_mod, experts, batch, inter, hid, top, dtype):
+    """Experts no row chose, more rows than a tile, duplicate pairs, pairs
+    that cancel, zero weights, NaN weight bytes, and pairs out of range."""
+    rng = np.random.default_rng(experts + batch)
+    items = [(*_fp8(inter, hid, 10 * e, nan_at=[(1, 2)] if e == 1 else ()), *_fp8(inter, hid, 10 * e + 1),
+              *_fp8(hid, inter, 10 * e + 2)) for e in range(experts)]
+    x = _x(batch, hid, 5, dtype)
+    pick = np.stack([rng.choice(max(experts - 1, top), top, replace=False) for _ in range(batch)])
+    pi, pr = pick.reshape(-1), np.repeat(np.arange(batch), top)
+    pw = rng.uniform(0.1, 1.0, pi.size).astype(np.float32)
+    pw[::7] = 0.0
+    pi = np.concatenate([pi, pi[:3], pi[3:4]])
+    pr = np.concatenate([pr, pr[:3], pr[3:4]])
+    pw = np.concatenate([pw, np.float32([0.5, 0.25, 0.125]), -pw[3:4]])
+    host = [tuple(t.cpu().numpy() for t in it) for it in items]
+    want = oracle_mod.fp8_mlp_many_pair_weighted(host, x.float().cpu().numpy(), pi, pr, pw)
+    args = [torch.from_numpy(a).cuda() for a in (pi.astype(np.int64), pr.astype(np.int64), pw)]
+    got = nat.fp8_e4m3_block_mlp_many_pair_weighted_f32(items, x, *args)
+    assert rel_l2(got.cpu().numpy(), want) < 2e-5
+    bad = [torch.cat([a, torch.tensor(v, dtype=a.dtype, device="cuda")])
+           for a, v in zip(args, ([experts, -1, 0], [0, 0, batch], [1.0, 1.0, 1.0]))]
+    out, n = nat.fp8_e4m3_block_mlp_many_pair_weighted_nosync(items, x, *bad)
+    assert int(n.item()) == 3 and torch.equal(out, got)
