@@ -722,6 +722,24 @@ int kv_dense_layer_decode_u16_ext_packed_rows8(
     uint16_t* out, int64_t hidden_size, int64_t intermediate_size, int64_t num_heads, int64_t num_kv_heads,
     float rms_eps, float rope_theta);
 
+/* A prompt of `rows` rows (hidden and out [rows][hidden_size]) through the
+ * layer, each row's k/v committed (the reference's prefill loop,
+ * fp16_kv_cache.cpp:1591-1673, over packed weights).  Up to 8 rows have the
+ * bits of that many decode steps; longer prompts take 128 rows at a time
+ * through each step where hidden_size and intermediate_size are multiples of
+ * 32, head_dim of 8 and the weights 16-byte aligned (else one row at a time):
+ * the same roundings to the session's type, sums in another order.  Codes as
+ * the decode step's, 4 when the rows do not fit the cache (nothing is done
+ * then). */
+int kv_dense_layer_prefill_u16_ext_packed_rows8(
+    void* handle, int64_t layer, const uint16_t* hidden, int64_t rows, const uint16_t* input_norm_weight,
+    const uint16_t* post_norm_weight, const uint16_t* q_weight_packed, const uint16_t* k_weight_packed,
+    const uint16_t* v_weight_packed, const uint16_t* o_weight_packed, const uint16_t* gate_weight_packed,
+    const uint16_t* up_weight_packed, const uint16_t* down_weight_packed, const uint16_t* q_bias,
+    const uint16_t* k_bias, const uint16_t* v_bias, const uint16_t* q_norm_weight, const uint16_t* k_norm_weight,
+    uint16_t* out, int64_t hidden_size, int64_t intermediate_size, int64_t num_heads, int64_t num_kv_heads,
+    float rms_eps, float rope_theta);
+
 /* The entry points over row-major (unpacked) weights that the reference's
  * KV loader binds unconditionally (native/__init__.py:2615-2745):
  * kv_attention_decode_fp16 (fp16_kv_cache.cpp:780-918),

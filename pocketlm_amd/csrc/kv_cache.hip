@@ -24,6 +24,8 @@
 // else reads or writes a few hundred KB.
 #include <algorithm>
 #include <cmath>
+#include <initializer_list>
+#include <type_traits>
 #include <vector>
 
 #include "row8.h"
@@ -83,24 +85,13 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
     return t;
 }
 
-// Per-head q/k RMSNorm (rms_norm_heads_inplace, 561-584), RoPE at `pos`
-// (apply_rope_one, 518-539), q kept in fp32, k and v rounded into cache row
-// `pos`.  One wave per head: blocks [0, nh) take q heads, [nh, nh + nkv) k/v.
+// One head at `pos`, by one wave: per-head q/k RMSNorm (rms_norm_heads_inplace,
+// 561-584), RoPE (apply_rope_one, 518-539); a query head is kept in fp32, a
+// key head is rounded into its cache row.
 template <bool BF16>
-__global__ __launch_bounds__(64) void qk_rope_append_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                            const float* __restrict__ v,
-                                                            const uint16_t* __restrict__ q_norm,
-                                                            const uint16_t* __restrict__ k_norm,
-                                                            float* __restrict__ q_rot, uint16_t* __restrict__ k_row,
-                                                            uint16_t* __restrict__ v_row, int nh, int hd, int64_t pos,
-                                                            float theta, float eps) {
+__device__ __forceinline__ void rope_head(const float* src, const uint16_t* nw, int hd, int64_t pos, float theta,
+                                          float eps, int lane, bool is_q, float* q_out, uint16_t* k_out) {
 #pragma clang fp contract(off)
-    const int head = blockIdx.x;
-    const int lane = threadIdx.x;
-    const bool is_q = head < nh;
-    const int kvh = head - nh;
-    const float* src = is_q ? q + static_cast<int64_t>(head) * hd : k + static_cast<int64_t>(kvh) * hd;
-    const uint16_t* nw = is_q ? q_norm : k_norm;
     float scale = 1.0f;
     if (nw != nullptr) {
         float s = 0.0f;
@@ -121,25 +112,42 @@ __global__ __launch_bounds__(64) void qk_rope_append_kernel(const float* __restr
         const float y0 = x0 * c - x1 * sn;
         const float y1 = x1 * c + x0 * sn;
         if (is_q) {
-            q_rot[static_cast<int64_t>(head) * hd + p] = y0;
-            q_rot[static_cast<int64_t>(head) * hd + p + half] = y1;
+            q_out[p] = y0;
+            q_out[p + half] = y1;
         } else {
-            k_row[static_cast<int64_t>(kvh) * hd + p] = wr16(y0, BF16);
-            k_row[static_cast<int64_t>(kvh) * hd + p + half] = wr16(y1, BF16);
+            k_out[p] = wr16(y0, BF16);
+            k_out[p + half] = wr16(y1, BF16);
         }
     }
     if ((hd & 1) != 0 && lane == 0) {  // an odd head keeps its last element unrotated
         float x = src[hd - 1];
         if (nw != nullptr) x = x * scale * rd16(nw[hd - 1], BF16);
         if (is_q) {
-            q_rot[static_cast<int64_t>(head) * hd + hd - 1] = x;
+            q_out[hd - 1] = x;
         } else {
-            k_row[static_cast<int64_t>(kvh) * hd + hd - 1] = wr16(x, BF16);
+            k_out[hd - 1] = wr16(x, BF16);
         }
     }
+}
+
+// q heads to q_rot, k and v into cache row `pos`.  One wave per head: blocks
+// [0, nh) take q heads, [nh, nh + nkv) k/v.
+template <bool BF16>
+__global__ __launch_bounds__(64) void qk_rope_append_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                            const float* __restrict__ v,
+                                                            const uint16_t* __restrict__ q_norm,
+                                                            const uint16_t* __restrict__ k_norm,
+                                                            float* __restrict__ q_rot, uint16_t* __restrict__ k_row,
+                                                            uint16_t* __restrict__ v_row, int nh, int hd, int64_t pos,
+                                                            float theta, float eps) {
+    const int head = blockIdx.x;
+    const int lane = threadIdx.x;
+    const bool is_q = head < nh;
+    const int64_t at = static_cast<int64_t>(is_q ? head : head - nh) * hd;
+    rope_head<BF16>((is_q ? q : k) + at, is_q ? q_norm : k_norm, hd, pos, theta, eps, lane, is_q, q_rot + at,
+                    k_row + at);
     if (!is_q)
-        for (int d = lane; d < hd; d += 64)
-            v_row[static_cast<int64_t>(kvh) * hd + d] = wr16(v[static_cast<int64_t>(kvh) * hd + d], BF16);
+        for (int d = lane; d < hd; d += 64) v_row[at + d] = wr16(v[at + d], BF16);
 }
 
 // Flash-decode partials.  Workgroup (kvh, sp) takes the TOK tokens
@@ -237,11 +245,20 @@ __host__ __device__ constexpr int split_sum_floats(int hd, int group, int hs, in
            ~3;
 }
 
-template <bool BF16, int G, int VD, int TOK>
+template <bool BF16, int G, int VD, int TOK, bool ROWS>
 __global__ __launch_bounds__(kAttnThreads) void attention_split_kernel(
     const float* __restrict__ q_rot, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     int64_t kv_width, int hd, int group, int64_t T, float scale, int vec, int slots, float* __restrict__ part,
     float* __restrict__ ml) {
+    // a prompt's query rows are the grid's layers: row z sees T + z tokens
+    if (ROWS) {
+        const int64_t row = blockIdx.z, heads = static_cast<int64_t>(gridDim.x) * group;
+        T += row;
+        if (static_cast<int64_t>(blockIdx.y) * TOK >= T) return;
+        q_rot += row * heads * hd;
+        part += row * heads * gridDim.y * hd;
+        ml += row * heads * gridDim.y * 2;
+    }
     constexpr int HS = G < 4 ? G : 4;         // head slices
     constexpr int HPL = G / HS;               // heads per lane in the score pass
     constexpr int NTG = kAttnThreads / (4 * HS);  // token groups in the score pass
@@ -481,23 +498,23 @@ __global__ __launch_bounds__(kAttnThreads) void attention_split_kernel(
 }
 
 // The launchers return false for a shape no kernel instance covers.
-template <bool BF16, int G, int TOK>
+template <bool BF16, int G, int TOK, bool ROWS>
 bool launch_split_t(int vd, dim3 grid, size_t lds, hipStream_t st, const float* q_rot, const uint16_t* kc,
                     const uint16_t* vc, int64_t kvw, int hd, int group, int64_t T, float scale, int vec, int slots,
                     float* part, float* ml) {
     if (vd <= 1) {
-        hipLaunchKernelGGL((attention_split_kernel<BF16, G, 1, TOK>), grid, dim3(kAttnThreads), lds, st, q_rot, kc, vc,
-                           kvw, hd, group, T, scale, vec, slots, part, ml);
+        hipLaunchKernelGGL((attention_split_kernel<BF16, G, 1, TOK, ROWS>), grid, dim3(kAttnThreads), lds, st, q_rot,
+                           kc, vc, kvw, hd, group, T, scale, vec, slots, part, ml);
         return true;
     }
     if (vd == 2) {
-        hipLaunchKernelGGL((attention_split_kernel<BF16, G, 2, TOK>), grid, dim3(kAttnThreads), lds, st, q_rot, kc, vc,
-                           kvw, hd, group, T, scale, vec, slots, part, ml);
+        hipLaunchKernelGGL((attention_split_kernel<BF16, G, 2, TOK, ROWS>), grid, dim3(kAttnThreads), lds, st, q_rot,
+                           kc, vc, kvw, hd, group, T, scale, vec, slots, part, ml);
         return true;
     }
     if constexpr (8 * (TOK * (G < 4 ? G : 4) / 64) <= 16) {  // K pieces per lane: 2 * VD per token
-        hipLaunchKernelGGL((attention_split_kernel<BF16, G, 4, TOK>), grid, dim3(kAttnThreads), lds, st, q_rot, kc, vc,
-                           kvw, hd, group, T, scale, vec, slots, part, ml);
+        hipLaunchKernelGGL((attention_split_kernel<BF16, G, 4, TOK, ROWS>), grid, dim3(kAttnThreads), lds, st, q_rot,
+                           kc, vc, kvw, hd, group, T, scale, vec, slots, part, ml);
         return true;
     }
     return false;
@@ -509,16 +526,16 @@ bool launch_split_g(int tok, int vd, dim3 grid, size_t lds, hipStream_t st, cons
                     float* part, float* ml) {
     if constexpr (G >= 4) {
         if (tok == 16)
-            return launch_split_t<BF16, G, 16>(vd, grid, lds, st, q_rot, kc, vc, kvw, hd, group, T, scale, vec, slots,
+            return launch_split_t<BF16, G, 16, false>(vd, grid, lds, st, q_rot, kc, vc, kvw, hd, group, T, scale, vec, slots,
                                                part, ml);
     }
     if constexpr (G >= 2) {
         if (tok == 32)
-            return launch_split_t<BF16, G, 32>(vd, grid, lds, st, q_rot, kc, vc, kvw, hd, group, T, scale, vec, slots,
+            return launch_split_t<BF16, G, 32, false>(vd, grid, lds, st, q_rot, kc, vc, kvw, hd, group, T, scale, vec, slots,
                                                part, ml);
     }
     if (tok != 64) return false;
-    return launch_split_t<BF16, G, 64>(vd, grid, lds, st, q_rot, kc, vc, kvw, hd, group, T, scale, vec, slots, part,
+    return launch_split_t<BF16, G, 64, false>(vd, grid, lds, st, q_rot, kc, vc, kvw, hd, group, T, scale, vec, slots, part,
                                        ml);
 }
 
@@ -573,6 +590,44 @@ bool launch_split(int tok, dim3 grid, size_t lds, hipStream_t st, const float* q
         default:
             return launch_split_g<BF16, kMaxGroup>(tok, vd, grid, lds, st, q_rot, kc, vc, kvw, hd, group, T, scale, vec,
                                                    slots, part, ml);
+    }
+}
+
+// The same for a prompt's query rows (grid.z of them): splits of the largest
+// size the kernel has for the shape, since the rows fill the compute units.
+template <bool BF16, int G>
+bool launch_split_rows_g(int tok, int vd, dim3 grid, size_t lds, hipStream_t st, const float* q_rot,
+                         const uint16_t* kc, const uint16_t* vc, int64_t kvw, int hd, int group, int64_t T,
+                         float scale, int vec, int slots, float* part, float* ml) {
+    if constexpr (G >= 4) {
+        if (tok == 32)
+            return launch_split_t<BF16, G, 32, true>(vd, grid, lds, st, q_rot, kc, vc, kvw, hd, group, T, scale, vec,
+                                                     slots, part, ml);
+    }
+    if (tok != 64) return false;
+    return launch_split_t<BF16, G, 64, true>(vd, grid, lds, st, q_rot, kc, vc, kvw, hd, group, T, scale, vec, slots,
+                                             part, ml);
+}
+
+int split_tokens_rows(int g, int hd) {
+    return split_vd(hd) == 4 && split_hs(g) == 4 ? kMaxSplitTokens / 2 : kMaxSplitTokens;
+}
+
+template <bool BF16>
+bool launch_split_rows(int tok, dim3 grid, size_t lds, hipStream_t st, const float* q_rot, const uint16_t* kc,
+                       const uint16_t* vc, int64_t kvw, int hd, int group, int64_t T, float scale, int vec, int slots,
+                       float* part, float* ml) {
+    const int vd = split_vd(hd);
+    auto run = [&](auto g) {
+        return launch_split_rows_g<BF16, decltype(g)::value>(tok, vd, grid, lds, st, q_rot, kc, vc, kvw, hd, group, T,
+                                                             scale, vec, slots, part, ml);
+    };
+    switch (split_g(group)) {
+        case 1: return run(std::integral_constant<int, 1>{});
+        case 2: return run(std::integral_constant<int, 2>{});
+        case 4: return run(std::integral_constant<int, 4>{});
+        case 8: return run(std::integral_constant<int, 8>{});
+        default: return run(std::integral_constant<int, kMaxGroup>{});
     }
 }
 
@@ -656,6 +711,44 @@ __global__ __launch_bounds__(kMergeThreads) void attention_merge_kernel(const fl
     }
 }
 
+// The merge for a prompt's query rows: one wave per (row blockIdx.y, head),
+// lanes over the splits for the weights, then over the head's dimensions.
+// Row y has the splits of its T + y tokens, of the launch's nsplit.
+__global__ __launch_bounds__(256) void attention_merge_rows_kernel(const float* __restrict__ part,
+                                                                  const float* __restrict__ ml,
+                                                                  float* __restrict__ context, int nh, int hd,
+                                                                  int group, int nsplit, int tok, int64_t T) {
+    constexpr int D = kMaxHeadDim / 64;  // dimensions per lane
+    const int lane = threadIdx.x & 63;
+    const int head = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (head >= nh) return;
+    const int64_t row = blockIdx.y;
+    const int ns = static_cast<int>((T + row + tok - 1) / tok);
+    const int kvh = head / group;
+    const int64_t base = (row * nh + static_cast<int64_t>(kvh) * group) * nsplit + head - kvh * group;
+    float m = -INFINITY;
+    for (int s = lane; s < ns; s += 64) m = fmaxf(m, ml[(base + static_cast<int64_t>(s) * group) * 2]);
+    m = seg_max<64>(m, lane);
+    float den = 0.0f, acc[D] = {};
+    for (int s0 = 0; s0 < ns; s0 += 64) {
+        const int n = min(ns - s0, 64);
+        const int64_t slot = base + static_cast<int64_t>(s0 + min(lane, n - 1)) * group;
+        const float w = lane < n ? expf(ml[slot * 2] - m) : 0.0f;
+        den += lane < n ? w * ml[slot * 2 + 1] : 0.0f;
+        for (int u = 0; u < n; ++u) {
+            const float wu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), u));
+            const float* p = part + (base + static_cast<int64_t>(s0 + u) * group) * hd;
+#pragma unroll
+            for (int d = 0; d < D; ++d)
+                if (lane + 64 * d < hd) acc[d] = fmaf(wu, p[lane + 64 * d], acc[d]);
+        }
+    }
+    den = seg_sum<64>(den, lane);
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (lane + 64 * d < hd) context[(row * nh + head) * hd + lane + 64 * d] = acc[d] / den;
+}
+
 // attention_out = storage(proj); resid = hidden + attention_out (fp32);
 // post = storage(rms_norm(storage(resid)) * w)   (1468-1491).
 template <bool BF16>
@@ -677,6 +770,224 @@ __global__ __launch_bounds__(kNormThreads) void post_attention_kernel(const uint
     const float scale = 1.0f / sqrtf(ms + eps);
     for (int i = threadIdx.x; i < n; i += blockDim.x)
         post[i] = wr16(rd16(wr16(resid[i], BF16), BF16) * scale * rd16(w[i], BF16), BF16);
+}
+
+// ------------------------------------------------------------------ prompt rows
+//
+// A prompt through the layer takes up to kRow8BatchRows rows at a time
+// through each step, so that every weight is read once for all of them
+// (120 rows one at a time: 120 times; 3584 / 18944 in fp16, 120 rows: 13.6 ->
+// 0.37 ms).  The projections run on the matrix
+// cores (row8_batch.hip) and leave sums per K slice, which the next kernel
+// adds; activations go to them as planes of 16-bit values in the order
+// row8.h describes.  The values that a row's step rounds to the
+// storage type are rounded the same here; sums run in another order.
+
+constexpr int kRowThreads = 1024;
+
+// Stores eight columns of row `row`, its piece (g, q) at 4 g + q, into a
+// plane of `tiles` token tiles (row8.h).
+__device__ __forceinline__ void store_piece(uint16_t* plane, int tiles, int64_t row, int64_t piece,
+                                            const uint32_t (&v)[8]) {
+    const int64_t at = ((piece >> 2) * tiles + (row >> 4)) * 64 + (piece & 3) * 16 + (row & 15);
+    reinterpret_cast<uint4*>(plane)[at] =
+        make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16));
+}
+
+// Column j of a row's piece.
+__device__ __forceinline__ int64_t piece_column(int64_t piece, int j) { return (piece >> 2) * 32 + 4 * j + (piece & 3); }
+
+// The workgroup's largest 32-bit value, returned to every thread.
+__device__ __forceinline__ uint32_t block_max(uint32_t v, uint32_t* red) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v = max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), off)));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    for (int w = 0; w < static_cast<int>(blockDim.x >> 6); ++w) v = max(v, red[w]);
+    __syncthreads();
+    return v;
+}
+
+// fp32 value -> its 16-bit parts, whose sum times `scale`'s inverse is the
+// value to 2^-24 of it (fp16: two parts rounded to nearest, the row scaled by
+// a power of two that puts its largest value at 2^14..2^15, so a part below
+// fp16's range is below 2^-40 of the row's largest value) or exactly (bf16:
+// three parts of 8 bits).  Infinities and NaNs stay whole in the first part.
+template <bool BF16>
+__device__ __forceinline__ void split_parts(float v, float scale, uint32_t (&p)[3]) {
+    if constexpr (BF16) {
+        const uint32_t b = __float_as_uint(v);
+        if ((b & 0x7F800000u) == 0x7F800000u) {
+            p[0] = (b & 0x007FFFFFu) != 0 ? 0x7FC0u : b >> 16;
+            p[1] = p[2] = 0;
+            return;
+        }
+        p[0] = b >> 16;
+        const float r1 = v - __uint_as_float(b & 0xFFFF0000u);
+        p[1] = __float_as_uint(r1) >> 16;
+        const float r2 = r1 - __uint_as_float(__float_as_uint(r1) & 0xFFFF0000u);
+        p[2] = __float_as_uint(r2) >> 16;
+    } else {
+        const float s = v * scale;
+        const _Float16 h = static_cast<_Float16>(s);
+        const float r = s - static_cast<float>(h);
+        p[0] = __builtin_bit_cast(uint16_t, h);
+        p[1] = r - r == 0.0f ? __builtin_bit_cast(uint16_t, static_cast<_Float16>(r)) : 0;
+    }
+}
+
+// The power of two for a row whose largest absolute value has these bits,
+// and its inverse.
+__device__ __forceinline__ float row_scale(uint32_t max_bits, float& inverse) {
+    const uint32_t e = min(max(max_bits >> 23, 16u), 254u);  // 254: the row holds an infinity or a NaN
+    inverse = __uint_as_float((e - 14u) << 23);
+    return __uint_as_float((268u - e) << 23);
+}
+
+// storage(rms_norm(hidden) * w) of each row, in pieces.
+template <bool BF16>
+__global__ __launch_bounds__(kRowThreads) void norm_rows_kernel(const uint16_t* __restrict__ hidden,
+                                                                const uint16_t* __restrict__ w,
+                                                                uint16_t* __restrict__ x, int tiles, int64_t n, float eps) {
+#pragma clang fp contract(off)
+    __shared__ float red[kRowThreads / 64];
+    const uint16_t* h = hidden + blockIdx.x * n;
+    float s = 0.0f;
+    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
+        const float v = rd16(h[i], BF16);
+        s += v * v;
+    }
+    const float scale = 1.0f / sqrtf(block_sum(s, red) / static_cast<float>(n) + eps);
+    for (int64_t p = threadIdx.x; p < n / 8; p += blockDim.x) {
+        uint32_t v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int64_t c = piece_column(p, j);
+            v[j] = wr16(rd16(h[c], BF16) * scale * rd16(w[c], BF16), BF16);
+        }
+        store_piece(x, tiles, blockIdx.x, p, v);
+    }
+}
+
+// Sum over the K slices of a projection's element.
+__device__ __forceinline__ float sum_slices(const float* part, int64_t at, int splits, int64_t stride) {
+    float v = part[at];
+    for (int s = 1; s < splits; ++s) v += part[at + s * stride];
+    return v;
+}
+
+// qk_rope_append_kernel for row blockIdx.y at position pos + blockIdx.y, from
+// the sums per K slice of the row [q | k | v], biases added.
+template <bool BF16>
+__global__ __launch_bounds__(64) void qk_rope_rows_kernel(const float* __restrict__ part, int splits, int64_t ld,
+                                                          const uint16_t* __restrict__ q_bias,
+                                                          const uint16_t* __restrict__ k_bias,
+                                                          const uint16_t* __restrict__ v_bias,
+                                                          const uint16_t* __restrict__ q_norm,
+                                                          const uint16_t* __restrict__ k_norm,
+                                                          float* __restrict__ q_rot, uint16_t* __restrict__ k_rows,
+                                                          uint16_t* __restrict__ v_rows, int nh, int nkv, int hd,
+                                                          int64_t pos, float theta, float eps) {
+    __shared__ float src[kMaxHeadDim];
+    const int head = blockIdx.x, lane = threadIdx.x;
+    const int64_t row = blockIdx.y, stride = gridDim.y * ld;
+    const bool is_q = head < nh;
+    const int64_t at = static_cast<int64_t>(is_q ? head : head - nh) * hd;
+    const int64_t H = static_cast<int64_t>(nh) * hd, kvw = static_cast<int64_t>(nkv) * hd;
+    const uint16_t* bias = is_q ? q_bias : k_bias;
+    for (int d = lane; d < hd; d += 64)
+        src[d] = sum_slices(part, row * ld + (is_q ? 0 : H) + at + d, splits, stride) +
+                 (bias != nullptr ? rd16(bias[at + d], BF16) : 0.0f);
+    if (!is_q)
+        for (int d = lane; d < hd; d += 64)
+            v_rows[row * kvw + at + d] =
+                wr16(sum_slices(part, row * ld + H + kvw + at + d, splits, stride) +
+                         (v_bias != nullptr ? rd16(v_bias[at + d], BF16) : 0.0f),
+                     BF16);
+    __syncthreads();
+    rope_head<BF16>(src, is_q ? q_norm : k_norm, hd, pos + row, theta, eps, lane, is_q, q_rot + row * H + at,
+                    k_rows + row * kvw + at);
+}
+
+// fp32 rows -> their parts, in pieces: the row itself, or (SILU) silu(gate) *
+// up of the sums per K slice of the row [gate | up], kept in `val` between
+// the two passes.
+template <bool BF16, bool SILU>
+__global__ __launch_bounds__(kRowThreads) void split_rows_kernel(const float* __restrict__ part, int splits,
+                                                                 int64_t ld, float* val, uint16_t* __restrict__ x,
+                                                                 float* __restrict__ inv, int tiles, int64_t n) {
+    __shared__ uint32_t red[kRowThreads / 64];
+    const int64_t row = blockIdx.x, rows = gridDim.x;
+    float* v = val + row * n;
+    float scale = 1.0f;
+    if (SILU || !BF16) {
+        uint32_t top = 0;
+        for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
+            if constexpr (SILU) {
+                const float g = sum_slices(part, row * ld + i, splits, rows * ld);
+                const float u = sum_slices(part, row * ld + n + i, splits, rows * ld);
+                v[i] = (g / (1.0f + expf(-g))) * u;
+            }
+            top = max(top, __float_as_uint(v[i]) & 0x7FFFFFFFu);
+        }
+        top = block_max(top, red);  // also orders the row's values before the pass below
+        if constexpr (!BF16) {
+            float inverse;
+            scale = row_scale(top, inverse);
+            if (threadIdx.x == 0) inv[row] = inverse;
+        }
+    }
+    constexpr int PL = plm::row8_planes(BF16);
+    for (int64_t p = threadIdx.x; p < n / 8; p += blockDim.x) {
+        uint32_t o[PL][8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            uint32_t t[3];
+            split_parts<BF16>(v[piece_column(p, j)], scale, t);
+#pragma unroll
+            for (int k = 0; k < PL; ++k) o[k][j] = t[k];
+        }
+#pragma unroll
+        for (int k = 0; k < PL; ++k) store_piece(x + k * tiles * 16 * n, tiles, row, p, o[k]);
+    }
+}
+
+// post_attention_kernel for row blockIdx.x, from the o projection's sums per
+// K slice; post permuted.
+template <bool BF16>
+__global__ __launch_bounds__(kRowThreads) void post_attention_rows_kernel(const uint16_t* __restrict__ hidden,
+                                                                          const float* __restrict__ part, int splits,
+                                                                          const uint16_t* __restrict__ w,
+                                                                          float* resid, uint16_t* __restrict__ post, int tiles,
+                                                                          int64_t n, float eps) {
+#pragma clang fp contract(off)
+    __shared__ float red[kRowThreads / 64];
+    const int64_t at = blockIdx.x * n, stride = gridDim.x * n;
+    float s = 0.0f;
+    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
+        const float r = rd16(hidden[at + i], BF16) + rd16(wr16(sum_slices(part, at + i, splits, stride), BF16), BF16);
+        resid[at + i] = r;
+        const float rq = rd16(wr16(r, BF16), BF16);
+        s += rq * rq;
+    }
+    const float scale = 1.0f / sqrtf(block_sum(s, red) / static_cast<float>(n) + eps);
+    for (int64_t p = threadIdx.x; p < n / 8; p += blockDim.x) {
+        uint32_t v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int64_t c = piece_column(p, j);
+            v[j] = wr16(rd16(wr16(resid[at + c], BF16), BF16) * scale * rd16(w[c], BF16), BF16);
+        }
+        store_piece(post, tiles, blockIdx.x, p, v);
+    }
+}
+
+// out = storage(resid + the down projection).
+template <bool BF16>
+__global__ __launch_bounds__(256) void add_rows_kernel(const float* __restrict__ resid, const float* __restrict__ part,
+                                                       int splits, uint16_t* __restrict__ out, int64_t n) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i < n) out[i] = wr16(resid[i] + sum_slices(part, i, splits, n), BF16);
 }
 
 struct LayerLengths {
@@ -859,6 +1170,166 @@ int dense_decode(KvSession* s, int64_t layer, const DenseArgs& a) {
     return plm::row8_gemv_x(x_act, &down, 1, I, dc, stream);
 }
 
+// The largest scratch the attention partials of a prompt's rows may take:
+// fewer query rows per attention launch beyond it.
+constexpr int64_t kPromptPartBytes = int64_t(64) << 20;
+
+// Rows of a prompt through the layer at once (m of them, at most
+// kRow8BatchRows): the same steps as dense_decode, each for all rows.  The
+// shape has passed dense_decode's checks.
+template <bool BF16>
+int dense_prompt_rows(KvSession* s, int64_t layer, const DenseArgs& a, int m) {
+    const int64_t H = a.hidden_size, I = a.inter, hd = H / a.nh, kvw = a.nkv * hd, group = a.nh / a.nkv;
+    LayerLengths& st = s->layers[static_cast<size_t>(layer)];
+    const int64_t pos = st.committed + st.tentative, T = pos + m;
+    const int g = split_g(static_cast<int>(group));
+    const int tok = split_tokens_rows(g, static_cast<int>(hd));
+    const int64_t nsplit = (T + tok - 1) / tok;
+    if (nsplit > kMaxSplits) return plm::fail(106, "context too long for one attention launch");
+    const int64_t row_part = a.nh * nsplit * hd * 4;
+    const int64_t arows = std::max<int64_t>(1, std::min<int64_t>(m, kPromptPartBytes / row_part));
+    constexpr int PL = plm::row8_planes(BF16);
+    const int64_t qkv_ld = H + 2 * kvw;
+    const int s_qkv = plm::row8_batch_splits(qkv_ld, H), s_o = plm::row8_batch_splits(H, H);
+    const int s_gu = plm::row8_batch_splits(2 * I, H), s_down = plm::row8_batch_splits(H, I);
+    const int64_t part_floats = m * std::max({s_qkv * qkv_ld, s_o * H, s_gu * 2 * I, s_down * H});
+    // workspace: x u16 planes | slices f32 | q_rot f32 | part | ml | ctx f32 | resid f32 | silu(gate) * up f32 | inv
+    const int64_t sz[] = {PL * plm::row8_plane_bytes(m, std::max(H, I)), part_floats * 4, m * H * 4, arows * row_part,
+                          arows * a.nh * nsplit * 8,   m * H * 4,       m * H * 4, m * I * 4,
+                          m * 4};
+    constexpr int nbuf = static_cast<int>(sizeof(sz) / sizeof(sz[0]));
+    size_t off[nbuf];
+    size_t total = 0;
+    for (int i = 0; i < nbuf; ++i) {
+        off[i] = total;
+        total += align256(static_cast<size_t>(sz[i]));
+    }
+    char* ws = static_cast<char*>(plm::workspace(total));
+    if (ws == nullptr) return plm::fail(108, "workspace");
+    uint16_t* x = reinterpret_cast<uint16_t*>(ws + off[0]);
+    float* slices = reinterpret_cast<float*>(ws + off[1]);
+    float* q_rot = reinterpret_cast<float*>(ws + off[2]);
+    float* part = reinterpret_cast<float*>(ws + off[3]);
+    float* ml = reinterpret_cast<float*>(ws + off[4]);
+    float* ctx = reinterpret_cast<float*>(ws + off[5]);
+    float* resid = reinterpret_cast<float*>(ws + off[6]);
+    float* act = reinterpret_cast<float*>(ws + off[7]);
+    float* inv = reinterpret_cast<float*>(ws + off[8]);
+    const hipStream_t stream = plm::current_stream();
+    const int tiles = plm::row8_token_tiles(m);
+    const dim3 per_row(static_cast<unsigned>(m)), row_block(kRowThreads);
+    int code = 0;
+
+    plm::Row8Batch b;
+    b.x = x;
+    b.part = slices;
+    b.m = m;
+    b.dtype_code = BF16 ? 1 : 0;
+    auto project = [&](std::initializer_list<plm::Row8BatchMat> mats, int64_t K, int64_t ld, int planes, int splits) {
+        b.nmats = 0;
+        for (const plm::Row8BatchMat& mat : mats) b.mats[b.nmats++] = mat;
+        b.K = K;
+        b.ld = ld;
+        b.planes = planes;
+        b.splits = splits;
+        b.inv = planes > 1 && !BF16 ? inv : nullptr;
+        return plm::row8_batch(b, stream);
+    };
+
+    hipLaunchKernelGGL((norm_rows_kernel<BF16>), per_row, row_block, 0, stream, a.hidden, a.input_norm, x, tiles, H, a.eps);
+    if ((code = plm::check_launch("input norm rows")) != 0) return code;
+    code = project({{a.q_w, H, 0}, {a.k_w, kvw, H}, {a.v_w, kvw, H + kvw}}, H, qkv_ld, 1, s_qkv);
+    if (code != 0) return code;
+    uint16_t* kc = s->k_rows(layer);
+    uint16_t* vc = s->v_rows(layer);
+    hipLaunchKernelGGL((qk_rope_rows_kernel<BF16>), dim3(static_cast<unsigned>(a.nh + a.nkv), static_cast<unsigned>(m)),
+                       dim3(64), 0, stream, slices, s_qkv, qkv_ld, a.q_bias, a.k_bias, a.v_bias, a.q_norm, a.k_norm,
+                       q_rot, kc + pos * kvw, vc + pos * kvw, static_cast<int>(a.nh), static_cast<int>(a.nkv),
+                       static_cast<int>(hd), pos, a.theta, a.eps);
+    if ((code = plm::check_launch("q/k rope and cache append, rows")) != 0) return code;
+    st.tentative += m;  // the rows are in the cache once the stream reaches here
+
+    const int slots = split_slots(static_cast<int>(hd), static_cast<int>(group), tok);
+    const size_t lds = split_lds_bytes(static_cast<int>(hd), static_cast<int>(group), tok, slots);
+    const float scale = 1.0f / std::sqrt(static_cast<float>(hd));
+    const int vec = hd % 8 == 0 && kvw % 8 == 0 && plm::aligned16(kc) && plm::aligned16(vc);
+    for (int64_t r0 = 0; r0 < m; r0 += arows) {
+        const int64_t rows = std::min<int64_t>(arows, m - r0);
+        const int64_t t0 = pos + r0 + 1;  // tokens the first of these rows sees
+        const int64_t ns = (t0 + rows - 1 + tok - 1) / tok;
+        if (!launch_split_rows<BF16>(tok, dim3(static_cast<unsigned>(a.nkv), static_cast<unsigned>(ns),
+                                               static_cast<unsigned>(rows)),
+                                     lds, stream, q_rot + r0 * H, kc, vc, kvw, static_cast<int>(hd),
+                                     static_cast<int>(group), t0, scale, vec, slots, part, ml))
+            return plm::fail(106, "no attention kernel for %d-token splits of head_dim %lld", tok,
+                             static_cast<long long>(hd));
+        if ((code = plm::check_launch("attention split rows")) != 0) return code;
+        hipLaunchKernelGGL(attention_merge_rows_kernel,
+                           dim3(static_cast<unsigned>((a.nh + 3) / 4), static_cast<unsigned>(rows)), dim3(256), 0,
+                           stream, part, ml, ctx + r0 * H, static_cast<int>(a.nh), static_cast<int>(hd),
+                           static_cast<int>(group), static_cast<int>(ns), tok, t0);
+        if ((code = plm::check_launch("attention merge rows")) != 0) return code;
+    }
+
+    hipLaunchKernelGGL((split_rows_kernel<BF16, false>), per_row, row_block, 0, stream,
+                       static_cast<const float*>(nullptr), 0, int64_t(0), ctx, x, inv, tiles, H);
+    if ((code = plm::check_launch("context parts")) != 0) return code;
+    if ((code = project({{a.o_w, H, 0}}, H, H, PL, s_o)) != 0) return code;
+    hipLaunchKernelGGL((post_attention_rows_kernel<BF16>), per_row, row_block, 0, stream, a.hidden, slices, s_o,
+                       a.post_norm, resid, x, tiles, H, a.eps);
+    if ((code = plm::check_launch("post attention norm rows")) != 0) return code;
+    if ((code = project({{a.gate_w, I, 0}, {a.up_w, I, I}}, H, 2 * I, 1, s_gu)) != 0) return code;
+    hipLaunchKernelGGL((split_rows_kernel<BF16, true>), per_row, row_block, 0, stream, slices, s_gu, 2 * I, act, x, inv,
+                       tiles, I);
+    if ((code = plm::check_launch("activation parts")) != 0) return code;
+    if ((code = project({{a.down_w, H, 0}}, I, H, PL, s_down)) != 0) return code;
+    hipLaunchKernelGGL((add_rows_kernel<BF16>), dim3(static_cast<unsigned>(plm::ceil_div(m * H, 256))), dim3(256), 0,
+                       stream, resid, slices, s_down, a.out, m * H);
+    return plm::check_launch("residual rows");
+}
+
+int commit_rows(KvSession* s, int64_t count) {
+    for (LayerLengths& st : s->layers) {
+        const int64_t take = std::min(count, st.tentative);
+        st.committed += take;
+        st.tentative -= take;
+    }
+    return 0;
+}
+
+// A prompt: every row through the layer, then committed.  Prompts of up to
+// kPromptDecodeRows rows go one row at a time, so that they have the bits of
+// decode steps (a verifier's draft; 8 rows 0.9 ms, 9 rows together 0.2 ms);
+// longer ones kRow8BatchRows at a time where the shape suits
+// the row kernels (whole 32-column steps, 16-byte K pieces).
+constexpr int64_t kPromptDecodeRows = 8;
+
+template <bool BF16>
+int dense_prefill(KvSession* s, int64_t layer, const DenseArgs& a, int64_t rows) {
+    const bool shape_ok = valid_layer(s, layer) && a.nh > 0 && a.nkv > 0 && a.hidden_size % a.nh == 0 &&
+                          a.nh % a.nkv == 0 && a.nkv * (a.hidden_size / a.nh) == s->kv_width &&
+                          a.nh / a.nkv <= kMaxGroup && a.hidden_size / a.nh <= kMaxHeadDim;
+    int dev = 0;
+    const bool here = hipGetDevice(&dev) == hipSuccess && s != nullptr && dev == s->device;
+    const bool aligned = plm::aligned16(a.q_w) && plm::aligned16(a.k_w) && plm::aligned16(a.v_w) &&
+                         plm::aligned16(a.o_w) && plm::aligned16(a.gate_w) && plm::aligned16(a.up_w) &&
+                         plm::aligned16(a.down_w);
+    const bool batched = rows > kPromptDecodeRows && shape_ok && here && aligned && a.hidden_size % 32 == 0 &&
+                         a.inter % 32 == 0 && (a.hidden_size / a.nh) % 8 == 0;
+    const int64_t step = batched ? plm::kRow8BatchRows : 1;
+    for (int64_t r0 = 0; r0 < rows; r0 += step) {
+        const int64_t m = std::min(step, rows - r0);
+        DenseArgs c = a;
+        c.hidden = a.hidden + r0 * a.hidden_size;
+        c.out = a.out + r0 * a.hidden_size;
+        const int code =
+            batched ? dense_prompt_rows<BF16>(s, layer, c, static_cast<int>(m)) : dense_decode<BF16>(s, layer, c);
+        if (code != 0) return code;
+        commit_rows(s, m);
+    }
+    return 0;
+}
+
 }  // namespace
 
 // ====================================================================== C ABI
@@ -916,12 +1387,7 @@ PLM_EXPORT int kv_append_tentative(void* handle, int64_t layer, const uint16_t* 
 PLM_EXPORT int kv_commit(void* handle, int64_t count) {
     KvSession* s = static_cast<KvSession*>(handle);
     if (s == nullptr || count < 0) return 1;
-    for (LayerLengths& st : s->layers) {
-        const int64_t take = std::min(count, st.tentative);
-        st.committed += take;
-        st.tentative -= take;
-    }
-    return 0;
+    return commit_rows(s, count);
 }
 
 PLM_EXPORT int kv_rollback(void* handle) {
@@ -1054,4 +1520,33 @@ PLM_EXPORT int kv_dense_layer_decode_u16_ext_packed_rows8(
                          out,             hidden_size,       intermediate_size, num_heads,       num_kv_heads,
                          rms_eps,         rope_theta};
     return s->dtype_code == 1 ? dense_decode<true>(s, layer, a) : dense_decode<false>(s, layer, a);
+}
+
+PLM_EXPORT int kv_dense_layer_prefill_u16_ext_packed_rows8(
+    void* handle, int64_t layer, const uint16_t* hidden, int64_t rows, const uint16_t* input_norm_weight,
+    const uint16_t* post_norm_weight, const uint16_t* q_weight_packed, const uint16_t* k_weight_packed,
+    const uint16_t* v_weight_packed, const uint16_t* o_weight_packed, const uint16_t* gate_weight_packed,
+    const uint16_t* up_weight_packed, const uint16_t* down_weight_packed, const uint16_t* q_bias,
+    const uint16_t* k_bias, const uint16_t* v_bias, const uint16_t* q_norm_weight, const uint16_t* k_norm_weight,
+    uint16_t* out, int64_t hidden_size, int64_t intermediate_size, int64_t num_heads, int64_t num_kv_heads,
+    float rms_eps, float rope_theta) {
+    plm::clear_error();
+    if (handle == nullptr || hidden == nullptr || input_norm_weight == nullptr || post_norm_weight == nullptr ||
+        q_weight_packed == nullptr || k_weight_packed == nullptr || v_weight_packed == nullptr ||
+        o_weight_packed == nullptr || gate_weight_packed == nullptr || up_weight_packed == nullptr ||
+        down_weight_packed == nullptr || out == nullptr)
+        return 1;
+    if (hidden_size <= 0 || intermediate_size <= 0 || rows <= 0) return 2;
+    if (hidden_size > 0x7FFFFFFF || intermediate_size > 0x7FFFFFFF) return plm::fail(2, "dimension too large");
+    KvSession* s = static_cast<KvSession*>(handle);
+    if (valid_layer(s, layer)) {
+        const LayerLengths& st = s->layers[static_cast<size_t>(layer)];
+        if (st.committed + st.tentative + rows > s->max_seq_len) return 4;
+    }
+    const DenseArgs a = {hidden,          input_norm_weight, post_norm_weight,  q_weight_packed, k_weight_packed,
+                         v_weight_packed, o_weight_packed,   gate_weight_packed, up_weight_packed, down_weight_packed,
+                         q_bias,          k_bias,            v_bias,            q_norm_weight,   k_norm_weight,
+                         out,             hidden_size,       intermediate_size, num_heads,       num_kv_heads,
+                         rms_eps,         rope_theta};
+    return s->dtype_code == 1 ? dense_prefill<true>(s, layer, a, rows) : dense_prefill<false>(s, layer, a, rows);
 }

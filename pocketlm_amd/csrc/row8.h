@@ -41,4 +41,46 @@ int row8_gemv(const uint16_t* hidden, const float* hidden_f32, const Row8Mat* ma
               hipStream_t st);
 int row8_gemv_x(const Row8X& x, const Row8Mat* mats, int n, int64_t K, int dtype_code, hipStream_t st);
 
+// ------------------------------------------------------------------ many rows (row8_batch.hip)
+//
+// Up to kRow8BatchRows activation rows against row8 weights on the matrix
+// cores.  The activations come as planes of storage-type values whose sum is
+// the row (one plane for fp16 / bf16 rows; fp32 rows as row8_planes parts),
+// in the order the lanes of the kernel read them: 16-byte pieces
+// [K / 32][token tile][q = 0..3][token of the tile], piece (g, q) of a row
+// being its columns 32 g + 4 j + q, j = 0..7 (one load of a lane's weights
+// holds one column of its 8 rows).
+constexpr int kRow8BatchRows = 128;
+constexpr int row8_planes(bool bf16) { return bf16 ? 3 : 2; }
+// 16-row token tiles of an activation plane (rows past m may hold anything).
+constexpr int row8_token_tiles(int64_t m) { return m <= 16 ? 1 : (m <= 32 ? 2 : (m <= 64 ? 4 : 8)); }
+constexpr int64_t row8_plane_bytes(int64_t m, int64_t K) { return K / 32 * row8_token_tiles(m) * 1024; }
+
+struct Row8BatchMat {
+    const uint16_t* packed;
+    int64_t rows;      // a multiple of 8
+    int64_t out_col;   // first column of the output
+    int64_t first_tile = 0;
+};
+
+// part[s][m][out_col + row] = sum over K slice s of x_m W[row], times
+// inv[m] when inv is set.
+struct Row8Batch {
+    Row8BatchMat mats[3];
+    int nmats = 0;
+    const uint16_t* x = nullptr;   // planes, row8_plane_bytes each
+    const float* inv = nullptr;
+    float* part = nullptr;         // [splits][m][ld]
+    int64_t ld = 0;                // a multiple of 4
+    int64_t K = 0;                 // a multiple of 32
+    int planes = 1;
+    int m = 0;                     // at most kRow8BatchRows
+    int splits = 1;                // of row8_batch_splits
+    int dtype_code = 0;
+};
+
+// K slices of a launch over `rows` weight rows in all.
+int row8_batch_splits(int64_t rows, int64_t K);
+int row8_batch(const Row8Batch& p, hipStream_t st);
+
 }  // namespace plm

@@ -1725,27 +1725,43 @@ class NativeKvSession:
         """src/pcketlm/native/__init__.py:3041-3120 ->
         kv_dense_layer_decode_u16_ext_packed_rows8 (fp16_kv_cache.cpp:1533).
         The new k/v row is appended as a tentative row of `layer`."""
+        x, tensors, scalars = self._dense_layer_args(
+            hidden, 1, input_norm_weight, post_norm_weight, q_weight_packed, k_weight_packed, v_weight_packed,
+            o_weight_packed, gate_weight_packed, up_weight_packed, down_weight_packed, hidden_size=hidden_size,
+            intermediate_size=intermediate_size, num_heads=num_heads, num_kv_heads=num_kv_heads, head_dim=head_dim,
+            rms_eps=rms_eps, rope_theta=rope_theta, q_bias=q_bias, k_bias=k_bias, v_bias=v_bias,
+            q_norm_weight=q_norm_weight, k_norm_weight=k_norm_weight)
+        out = torch.empty((int(hidden_size),), dtype=self.dtype, device=self.device)
+        with _launch(self._lib, self.device):
+            code = self._lib.kv_dense_layer_decode_u16_ext_packed_rows8(
+                self._handle, int(layer), _p(x), *[_p(t) for t in tensors], _p(out), *scalars)
+        _check("kv_dense_layer_decode_u16_ext_packed_rows8", code)
+        return out
+
+    def _dense_layer_args(self, hidden, rows, input_norm_weight, post_norm_weight, *packed, hidden_size,
+                          intermediate_size, num_heads, num_kv_heads, head_dim=None, rms_eps, rope_theta, q_bias=None,
+                          k_bias=None, v_bias=None, q_norm_weight=None, k_norm_weight=None):
+        """The checks of a dense layer call: (hidden on the session's device,
+        the other tensors in the C ABI's order, the sizes and constants)."""
         raw = [hidden, input_norm_weight, post_norm_weight]
         if any(t.dtype != self.dtype for t in raw):
             raise TypeError(f"dense_layer_decode_packed_rows8 requires {self.dtype} raw tensors")
-        packed = [q_weight_packed, k_weight_packed, v_weight_packed, o_weight_packed, gate_weight_packed,
-                  up_weight_packed, down_weight_packed]
         if any(t.dtype != torch.uint16 for t in packed):
             raise TypeError("packed dense layer weights must be torch.uint16")
         if head_dim is not None and int(head_dim) * int(num_heads) != int(hidden_size):
             raise ValueError("head_dim must equal hidden_size // num_heads for this entry point")
         dev = self.device
-        raw_d = [_on(t, dev).reshape(-1) for t in raw]
-        if raw_d[0].numel() != int(hidden_size):
-            raise ValueError("hidden length does not match hidden_size")
         H, inter, kvw = int(hidden_size), int(intermediate_size), self.kv_width
+        raw_d = [_on(t, dev).reshape(-1) for t in raw]
+        if raw_d[0].numel() != rows * H:
+            raise ValueError("hidden length does not match hidden_size")
         if int(num_heads) <= 0 or H % int(num_heads) != 0:
             raise ValueError("hidden_size must be a multiple of num_heads")
         hd = H // int(num_heads)
-        if any(t.numel() != H for t in raw_d):
+        if any(t.numel() != H for t in raw_d[1:]):
             raise ValueError("hidden and norm weights must hold hidden_size values")
         packed_d = [_on(t, dev) for t in packed]
-        blocks = lambda rows: (rows + 7) // 8 * 8  # noqa: E731
+        blocks = lambda n: (n + 7) // 8 * 8  # noqa: E731
         want = [blocks(H) * H, blocks(kvw) * H, blocks(kvw) * H, blocks(H) * H, blocks(inter) * H,
                 blocks(inter) * H, blocks(H) * inter]
         if [t.numel() for t in packed_d] != want:
@@ -1755,24 +1771,25 @@ class NativeKvSession:
         for t, n in zip(opt, (H, kvw, kvw, hd, hd)):
             if t is not None and (t.numel() != n or t.dtype != self.dtype):
                 raise ValueError(f"biases and q/k norm weights must be {self.dtype} of the layer's sizes")
-        out = torch.empty((int(hidden_size),), dtype=self.dtype, device=dev)
-        with _launch(self._lib, dev):
-            code = self._lib.kv_dense_layer_decode_u16_ext_packed_rows8(
-                self._handle, int(layer), *[_p(t) for t in raw_d], *[_p(t) for t in packed_d],
-                *[_p(t) for t in opt], _p(out), int(hidden_size), int(intermediate_size), int(num_heads),
-                int(num_kv_heads), float(rms_eps), float(rope_theta))
-        _check("kv_dense_layer_decode_u16_ext_packed_rows8", code)
-        return out
+        return (raw_d[0], [*raw_d[1:], *packed_d, *opt],
+                (H, inter, int(num_heads), int(num_kv_heads), float(rms_eps), float(rope_theta)))
 
     def dense_layer_prefill_packed_rows8(self, layer: int, hidden: torch.Tensor, *weights: torch.Tensor,
                                          **kwargs) -> torch.Tensor:
         """kv_dense_layer_prefill_u16_ext's loop (fp16_kv_cache.cpp:1591-1673)
-        over the packed decode: each row is decoded, then committed."""
+        over the packed weights: every row decoded, then committed.  Up to 8
+        rows have the bits of that many decode steps; longer prompts go
+        through each step together (the same roundings, sums in another
+        order)."""
         rows = hidden.reshape(-1, int(kwargs["hidden_size"]))
         if self.committed_length(layer) + self.tentative_length(layer) + rows.shape[0] > self.max_seq_len:
             raise RuntimeError("kv_dense_layer_prefill failed with code 4 (cache full)")
-        outs = []
-        for row in rows:
-            outs.append(self.dense_layer_decode_packed_rows8(layer, row, *weights, **kwargs))
-            self.commit(1)
-        return torch.stack(outs)
+        if not rows.shape[0]:
+            raise RuntimeError("dense_layer_prefill_packed_rows8 needs at least one row")
+        x, tensors, scalars = self._dense_layer_args(rows, int(rows.shape[0]), *weights, **kwargs)
+        out = torch.empty(tuple(rows.shape), dtype=self.dtype, device=self.device)
+        with _launch(self._lib, self.device):
+            code = self._lib.kv_dense_layer_prefill_u16_ext_packed_rows8(
+                self._handle, int(layer), _p(x), int(rows.shape[0]), *[_p(t) for t in tensors], _p(out), *scalars)
+        _check("kv_dense_layer_prefill_u16_ext_packed_rows8", code)
+        return out
