@@ -50,6 +50,10 @@ unsigned* stream_words();
 // Number of compute units of the current device (cached).
 int cu_count();
 
+// Kernels whose LDS passes 64 KiB must say so once per device: bytes is the
+// most dynamic LDS a launch of fn asks for (its static LDS comes on top).
+int allow_large_lds(const void* fn, int bytes);
+
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }

@@ -8,6 +8,16 @@
 
 namespace plm {
 
+constexpr int kPanelOuts = 8;     // weights of one fp8_panel_linear call
+// Activation rows from which the panel kernel is the faster one, for a launch
+// over `rows` weight rows.  The skinny kernel's time grows with the rows (us,
+// bf16 / fp32 at 32, 64 and 128 rows: 7168x16384 53 / 80, 80 / 157, 155 / 310;
+// 2048x7168 25 / 39, 38 / 39, 39 / 39), the panel kernel's hardly does
+// (105 / 88, 23 / 23): they cross at about 80 / 36 rows of a tall weight and
+// 32 / 14 of a short one, 68 / 36 for 24576x1536.
+constexpr int64_t panel_from(int64_t rows, bool bf16) {
+    return bf16 ? (rows >= 4096 ? 65 : 33) : (rows >= 4096 ? 33 : 17);
+}
 constexpr int kBatchGroups = 64;  // weights per launch (their addresses travel as kernel arguments)
 
 // Where the tokens of a grouped launch are, on the device (all indexed by
@@ -42,9 +52,18 @@ struct BatchRows {
     int waves = 0;                      // K blocks b = w, w + waves, ... are wave w's
     bool tiled = false;                 // weights in 8-row tiles
     BatchGroups groups;
+    // fp8_panel_linear: the weights w[0][i] of out_rows[i] rows each, to outs[i]
+    float* outs[kPanelOuts] = {};
+    int64_t out_rows[kPanelOuts] = {};
 };
 
 int fp8_batch_rows(const BatchRows& p, hipStream_t st);
+
+// Prompt chunks (fp8_panel_kernel), the same bits: several linears over one
+// packed copy of the activations, and the SwiGLU MLP (gate_up's two weights,
+// then down's).
+int fp8_panel_linear(const BatchRows& p, int outs, hipStream_t st);
+int fp8_panel_mlp(const BatchRows& gate_up, const BatchRows& down, hipStream_t st);
 
 // Waves of the down phase over nb K blocks (one group's): see fp8_down_kernel.
 constexpr int kBatchDownWaves = 16;

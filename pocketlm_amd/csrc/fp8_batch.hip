@@ -14,10 +14,10 @@
 // and then waves are added in the same order: a row's result has the bits of
 // a one-row call.
 //
-// Measured on an MI355X against passes of 8 rows: 24576x1536 at 509 bf16 rows
-// 787 -> 289 us, the 7168/2048 MLP at 256 fp32 rows 991 -> 251 us, 96 rows of
-// top-8 over 256 experts of 7168/2048 27.2 -> 2.02 ms (5.3 TB/s: the weights
-// of every chosen expert, read once).
+// Measured on an MI355X against passes of 8 rows: 7168x16384 at 16 bf16 rows
+// 52 -> 40 us, at 64 rows 226 -> 78 us; 96 rows of top-8 over 256 experts of
+// 7168/2048 27.2 -> 2.02 ms (5.3 TB/s: the weights of every chosen expert,
+// read once).
 #include <algorithm>
 #include <cstring>
 #include <type_traits>
@@ -390,6 +390,473 @@ __global__ __launch_bounds__(kPairThreads) void pair_sum_kernel(const float* __r
         for (int j = 0; j < 4; ++j) out[m * hid + col + j] = acc[j];
 }
 
+// ------------------------------------------------------------------ prompt chunks
+//
+// fp8_panel_kernel: a workgroup of 4 WR waves owns 64 WR weight rows and 8
+// column tiles of 16 (128 bf16 activation rows, or 64 rows as hi and lo).
+// The block's weights (as bytes, NaN bytes zeroed) and activations go through
+// LDS in the order the MFMA operands are read, double buffered, the next
+// block's loads in flight meanwhile: a weight byte is read once per 64 to 128
+// activation rows and an activation once per 64 to 128 weight rows.  Wave
+// (wr, wc) computes 32 rows by 4 column tiles.  The K blocks run in the order
+// of the skinny kernel's waves: the blocks of one wave into the two halves'
+// accumulators, which are then added to the total, so the sums are the same
+// bits.
+//
+// What bounds it: a wave's own instructions (at one to two waves per SIMD
+// conversions, scaling FMAs, MFMAs and LDS reads hardly overlap; more
+// workgroups per compute unit, deeper prefetch or single buffers changed
+// nothing).  24576x1536 at 509 bf16 rows: 289 us with the skinny kernel, 75
+// here (510 TFLOP/s) and 5 for packing; the 7168 / 2048 MLP at 256 fp32 rows
+// 251 -> 107 us (gate + up 74, down 38).
+//
+// The activations come packed ([block][column tile][half][piece][lane]
+// [8 values], kTileBytes per column tile and block) by fp8_pack_rows_kernel,
+// or from the gate/up launch's epilogue.  Rows past m hold anything (their
+// columns are dropped); columns past K are zero.
+
+constexpr int kPanelCols = 8;      // column tiles per workgroup
+constexpr int kTileBytes = 4096;   // one column tile of one block
+
+struct PanelArgs {
+    const uint8_t* w[2];
+    const float* s[2];
+    const char* x;
+    float* out;
+    char* xout;  // SILU: the packed hi / lo columns of silu(gate) * up
+    int64_t rows;
+    int64_t K;
+    int64_t scale_cols;
+    int64_t m;
+    int nblocks;
+    int waves;      // K slots
+    int row_tiles;  // workgroups along the rows
+    int col_tiles;  // workgroups along the activation rows
+    int out_tiles;  // SILU: column tiles of xout
+    int x_tiles;    // column tiles of x
+    int tiled;
+    // The K slots dealt to `splits` workgroups a tile (slot k to part k %
+    // splits): every slot's sums go to part[slot][m][part_ld] and a second
+    // kernel adds them in order.  1: the workgroup adds them itself.
+    int splits;
+    float* part;
+    int64_t part_ld;
+};
+
+// Byte offset of column `col` of activation row `li` of column tile `tile`.
+__device__ __forceinline__ int64_t packed_at(int64_t col, int tiles, int tile, int li) {
+    return ((col >> 7) * tiles + tile) * kTileBytes + ((col >> 6) & 1) * 2048 + ((col >> 3) & 1) * 1024 +
+           (((col >> 4) & 3) * 16 + li) * 16 + (col & 7) * 2;
+}
+
+// WR: 64 weight rows each (two wave rows of 32); MODE: bf16 activations
+// (kXBf16), fp32 ones as hi and lo in one chain (kXF32), or planes with
+// accumulators of their own (kXPlanes).
+template <int WR, bool SILU, int MODE, bool SPLIT>
+__global__ __launch_bounds__(256 * WR, 2) void fp8_panel_kernel(const PanelArgs a) {
+    constexpr int NW = 4 * WR;                    // waves: 2 WR along the rows, 2 along the columns
+    constexpr int CT = MODE == kXBf16 ? 4 : 2;    // token tiles per wave
+    constexpr int PL = MODE == kXPlanes ? 2 : 1;  // accumulator planes
+    constexpr int ABYTES = 4 * WR * 2048;         // a block's weights
+    constexpr int XBYTES = kPanelCols * kTileBytes;
+    constexpr int XL = XBYTES / (NW * 1024);      // activation loads per lane and block
+    constexpr int DEPTH = WR == 1 && MODE != kXPlanes ? 2 : 1;  // blocks in flight in registers
+    constexpr int STAGES = MODE == kXPlanes ? 1 : 2;            // blocks in LDS
+    extern __shared__ char panel[];               // [STAGES][ABYTES + XBYTES]
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, li = lane & 15, qd = lane >> 4;
+    const int wr = wave / 2, wc = wave % 2;
+    // workgroup -> tile: the column tiles of a row tile follow each other on one XCD
+    const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
+    const int rt = (seq / a.col_tiles) * 8 + xcd, ct = seq % a.col_tiles;
+    if (rt >= a.row_tiles) return;
+    constexpr int ROWS = SILU ? 32 * WR : 64 * WR;  // rows of one weight
+    const int64_t row0 = static_cast<int64_t>(rt) * ROWS;
+    const int64_t K = a.K;
+    const int nb = a.nblocks, nw = a.waves;
+
+    // the 16-row tile this wave loads: tiles 2 wr + t are wave row wr's; SILU: t = 0 gate, 1 up
+    const int64_t my_row = min(row0 + (SILU ? 16 * (wave / 2) : 16 * wave) + li, a.rows - 1);  // past the end: dropped
+    const uint8_t* wrow = (SILU && (wave & 1) ? a.w[1] : a.w[0]) +
+                          (a.tiled ? (my_row >> 3) * nb * 1024 + (my_row & 7) * 128 : my_row * K);
+    const float* sp[2];
+    sp[0] = a.s[0] + (row0 >> 7) * a.scale_cols;
+    sp[1] = SILU ? a.s[1] + (row0 >> 7) * a.scale_cols : sp[0];
+    const char* xsrc = a.x + static_cast<int64_t>(ct) * XBYTES + threadIdx.x * 16;
+    const int64_t xstep = static_cast<int64_t>(a.x_tiles) * kTileBytes;
+
+    // DEPTH blocks in flight in registers; the scales by vector loads: a
+    // scalar load in flight would hold up every LDS read (they share a counter
+    // and scalar loads return out of order)
+    plm_u32x4 wq[DEPTH][2], xq[DEPTH][XL];
+    float snext[DEPTH][2];
+    int vzero = 0;
+    asm("" : "+v"(vzero));
+    // the block after b in the order of this workgroup's K slots (nb: none)
+    const int first = SPLIT ? blockIdx.y : 0, step = SPLIT ? a.splits : 1;
+    auto after = [&](int b) { return b + nw < nb ? b + nw : (b % nw + step < nw ? b % nw + step : nb); };
+    int fb;  // the next block to fetch
+    auto fetch = [&](int u) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            // past the end of a row: its last 16 bytes, against zero activations
+            const int64_t off = min(static_cast<int64_t>(fb) * 128 + 64 * h + 16 * qd, K - 16);
+            wq[u][h] = xload16(wrow + (a.tiled ? off + (off >> 7) * 896 : off));
+        }
+#pragma unroll
+        for (int i = 0; i < XL; ++i) xq[u][i] = xload16(xsrc + fb * xstep + i * NW * 1024);
+        snext[u][0] = plm_gload_f32(sp[0] + fb + vzero);
+        if (SILU) snext[u][1] = plm_gload_f32(sp[1] + fb + vzero);
+        fb = after(fb);
+    };
+    // D: lane (activation row li, weight rows 4 qd + j)
+    auto token_tile = [&](int c) { return (ct * kPanelCols + wc * 4) / (MODE == kXBf16 ? 1 : 2) + c; };
+    // 4 floats at `row` of an output row of a.rows, the last of them perhaps past its end
+    auto store_row = [&](float* out, int64_t row, plm_f32x4 v) {
+        if (row + 4 <= a.rows && (reinterpret_cast<uintptr_t>(out + row) & 15) == 0) {
+            *reinterpret_cast<plm_f32x4*>(out + row) = v;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (row + j < a.rows) out[row + j] = v[j];
+        }
+    };
+    plm_f32x4 acc[2][PL][2][CT], total[2][CT];
+    bool bad = false;  // a NaN among the sums of an activation row
+    auto store_part = [&](int slot, int t, int c, plm_f32x4 v) {
+        const int64_t t_row = static_cast<int64_t>(token_tile(c)) * 16 + li;
+        if (t_row >= a.m) return;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bad = bad || v[j] != v[j];
+        // SILU: gate in columns 0 .., up in part_ld / 2 ..
+        store_row(a.part + (slot * a.m + t_row) * a.part_ld + (SILU && t ? a.part_ld / 2 : 0),
+                  row0 + (SILU ? 16 * wr : 32 * wr + 16 * t) + 4 * qd, v);
+    };
+    int stage = 0, cb;  // cb: the block being computed
+    // A block: its operands to LDS, the loads of the block DEPTH further, its products.
+    auto block = [&](int u, bool zero_nans) {
+        char* as = panel + stage * (ABYTES + XBYTES);
+        char* xs = as + ABYTES;
+        if (STAGES == 1) __syncthreads();  // the last block's reads
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            *reinterpret_cast<plm_u32x4*>(as + (wave * 2 + h) * 1024 + lane * 16) =
+                zero_nans ? zero_nan_bytes(wq[u][h]) : wq[u][h];
+#pragma unroll
+        for (int i = 0; i < XL; ++i)
+            *reinterpret_cast<plm_u32x4*>(xs + i * NW * 1024 + threadIdx.x * 16) = xq[u][i];
+        float sc[2];
+        sc[0] = lane_value(snext[u][0], 0);
+        sc[1] = SILU ? lane_value(snext[u][1], 0) : sc[0];
+        if (cb < nw) {  // a slot's first block
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int pl = 0; pl < PL; ++pl)
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+#pragma unroll
+                        for (int c = 0; c < CT; ++c) acc[h][pl][t][c] = plm_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+        if (fb < nb) fetch(u);
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            plm_bf16x8 a0[2], a1[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                weights_to_bf16(*reinterpret_cast<const plm_u32x4*>(as + ((wr * 2 + t) * 2 + h) * 1024 + lane * 16),
+                                a0[t], a1[t]);
+            auto operand = [&](int c, int p) {  // of the wave's column tile c, piece p
+                return *reinterpret_cast<const plm_bf16x8*>(xs + (wc * 4 + c) * kTileBytes + h * 2048 + p * 1024 +
+                                                            lane * 16);
+            };
+            auto add = [&](plm_f32x4& to, plm_f32x4 d, float f) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) to[j] = fmaf(d[j], f, to[j]);
+            };
+            const plm_f32x4 none = {0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (MODE == kXF32) {
+#pragma unroll
+                for (int c = 0; c < CT; ++c) {
+                    const plm_bf16x8 h0 = operand(2 * c, 0), h1 = operand(2 * c, 1);
+                    const plm_bf16x8 l0 = operand(2 * c + 1, 0), l1 = operand(2 * c + 1, 1);
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        plm_f32x4 d = mfma_bf16(a0[t], h0, none);
+                        d = mfma_bf16(a1[t], h1, d);
+                        d = mfma_bf16(a0[t], l0, d);
+                        d = mfma_bf16(a1[t], l1, d);
+                        add(acc[h][0][t][c], d, sc[SILU ? t : 0]);
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const plm_bf16x8 b0 = operand(c, 0), b1 = operand(c, 1);
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        plm_f32x4 d = mfma_bf16(a0[t], b0, none);
+                        d = mfma_bf16(a1[t], b1, d);
+                        add(MODE == kXPlanes ? acc[h][c % PL][t][c / 2] : acc[h][0][t][c % CT], d, sc[SILU ? t : 0]);
+                    }
+                }
+            }
+        }
+        if (cb + nw >= nb) {  // the slot's last block
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int c = 0; c < CT; ++c) {
+                    plm_f32x4 v = acc[0][0][t][c] + acc[1][0][t][c];
+                    if constexpr (PL == 2) v = v + (acc[0][1][t][c] + acc[1][1][t][c]);
+                    if constexpr (SPLIT)
+                        store_part(cb % nw, t, c, v);
+                    else
+                        total[t][c] = total[t][c] + v;
+                }
+        }
+        if (STAGES == 2) stage ^= 1;
+        cb = after(cb);
+    };
+    auto pass = [&](bool zero_nans) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int c = 0; c < CT; ++c) total[t][c] = plm_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        fb = cb = first;
+#pragma unroll
+        for (int u = 0; u < DEPTH; ++u)
+            if (fb < nb) fetch(u);
+        while (cb < nb) {
+#pragma unroll
+            for (int u = 0; u < DEPTH; ++u)
+                if (cb < nb) block(u, zero_nans);
+        }
+    };
+    pass(false);
+    if constexpr (!SPLIT) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    bad = bad || (total[t][c][j] != total[t][c][j] && token_tile(c) * 16 + li < a.m);
+    }
+    // NaN weight bytes count as 0: the blocks again (rows without one come out the same)
+    if (__syncthreads_or(bad)) pass(true);
+    if constexpr (SPLIT) return;
+
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        const int tile = token_tile(c);
+        const int64_t t_row = static_cast<int64_t>(tile) * 16 + li;
+        if constexpr (SILU) {
+            if (tile >= a.out_tiles / 2) continue;
+            // 4 of the 16 columns (row0 + 16 wr ..) of the down phase's activations
+            const int64_t col = row0 + 16 * wr + 4 * qd;
+            uint32_t hi[4], lo[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                split_f32<true>(__float_as_uint(plm_silu_mul(total[0][c][j], total[1][c][j])), hi[j], lo[j]);
+                if (col + j >= a.rows) hi[j] = lo[j] = 0u;
+            }
+            char* o = a.xout + packed_at(col, a.out_tiles, 2 * tile, li);
+            *reinterpret_cast<uint2*>(o) = make_uint2(hi[0] | (hi[1] << 16), hi[2] | (hi[3] << 16));
+            *reinterpret_cast<uint2*>(o + kTileBytes) = make_uint2(lo[0] | (lo[1] << 16), lo[2] | (lo[3] << 16));
+        } else if (t_row < a.m) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                store_row(a.out + t_row * a.rows, row0 + 32 * wr + 16 * t + 4 * qd, total[t][c]);
+        }
+    }
+}
+
+// The slots' sums of a split launch, added in order.
+__global__ __launch_bounds__(256) void fp8_panel_sum_kernel(const float* __restrict__ part, int slots, int64_t n,
+                                                            float* __restrict__ out) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= n) return;
+    float v = 0.0f;
+    for (int k = 0; k < slots; ++k) v += part[k * n + i];
+    out[i] = v;
+}
+
+// The same for gate and up (rows [gate | up] of ld columns), with the SiLU
+// epilogue: one thread per activation row and 8 columns of the packed
+// intermediate.
+__global__ __launch_bounds__(256) void fp8_panel_silu_kernel(const float* __restrict__ part, int slots, int64_t m,
+                                                             int64_t ld, int64_t rows, char* __restrict__ xout,
+                                                             int out_tiles, int64_t pieces) {
+    const int64_t id = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const int64_t t_row = id / pieces, col = (id - t_row * pieces) * 8;
+    if (t_row >= m) return;
+    float g[8], u[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) g[j] = u[j] = 0.0f;
+    if (col < rows)  // rows is a multiple of 16
+        for (int k = 0; k < slots; ++k) {
+            const float* p = part + (k * m + t_row) * ld + col;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                g[j] += p[j];
+                u[j] += p[ld / 2 + j];
+            }
+        }
+    uint32_t hi[8], lo[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        split_f32<true>(__float_as_uint(plm_silu_mul(g[j], u[j])), hi[j], lo[j]);
+        if (col >= rows) hi[j] = lo[j] = 0u;
+    }
+    char* o = xout + packed_at(col, out_tiles, static_cast<int>(t_row >> 4) * 2, static_cast<int>(t_row & 15));
+    *reinterpret_cast<uint4*>(o) = make_uint4(hi[0] | (hi[1] << 16), hi[2] | (hi[3] << 16), hi[4] | (hi[5] << 16),
+                                              hi[6] | (hi[7] << 16));
+    *reinterpret_cast<uint4*>(o + kTileBytes) = make_uint4(lo[0] | (lo[1] << 16), lo[2] | (lo[3] << 16),
+                                                           lo[4] | (lo[5] << 16), lo[6] | (lo[7] << 16));
+}
+
+// Activation rows packed for fp8_panel_kernel: one wave per (block, half,
+// token tile); fp32 rows as the column tiles 2 t (hi) and 2 t + 1 (lo).
+template <bool XB>
+__global__ __launch_bounds__(256) void fp8_pack_rows_kernel(const char* __restrict__ x, char* __restrict__ out,
+                                                            int64_t m, int64_t K, int64_t stride, int token_tiles,
+                                                            int x_tiles, int nblocks) {
+    const int64_t id = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const int h = id & 1;
+    const int64_t tile = (id >> 1) % token_tiles, b = (id >> 1) / token_tiles;
+    if (b >= nblocks) return;
+    const int64_t row = tile * 16 + (lane & 15), col = b * 128 + 64 * h + 16 * (lane >> 4);
+    if (row >= m) return;
+    plm_u32x4 hi[2] = {}, lo[2] = {};
+    if (col < K) {  // K is a multiple of 16
+        const char* src = x + row * stride + col * (XB ? 2 : 4);
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            if constexpr (XB) {
+                hi[p] = xload16(src + 16 * p);
+            } else {
+                plm_bf16x8 vh, vl;
+                split8<true>(xload16(src + 32 * p), xload16(src + 32 * p + 16), vh, vl);
+                hi[p] = __builtin_bit_cast(plm_u32x4, vh);
+                lo[p] = __builtin_bit_cast(plm_u32x4, vl);
+            }
+        }
+    }
+    char* o = out + (b * x_tiles + tile * (XB ? 1 : 2)) * kTileBytes + h * 2048 + lane * 16;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        *reinterpret_cast<plm_u32x4*>(o + p * 1024) = hi[p];
+        if (!XB) *reinterpret_cast<plm_u32x4*>(o + kTileBytes + p * 1024) = lo[p];
+    }
+}
+
+// Column tiles of m activation rows (two per token tile for hi and lo), in
+// whole workgroups.
+int panel_tiles(int64_t m, bool one_plane) {
+    return static_cast<int>(plm::ceil_div(plm::ceil_div(m, 16) * (one_plane ? 1 : 2), kPanelCols)) * kPanelCols;
+}
+
+int64_t panel_bytes(int64_t m, int64_t K, bool one_plane) {
+    return plm::ceil_div(K, 128) * panel_tiles(m, one_plane) * kTileBytes;
+}
+
+int pack_rows(const float* x, const uint16_t* xb, int64_t m, int64_t K, int64_t stride, char* out, hipStream_t st) {
+    const int token_tiles = static_cast<int>(plm::ceil_div(m, 16));
+    const int nb = static_cast<int>(plm::ceil_div(K, 128));
+    const dim3 grid(static_cast<unsigned>(plm::ceil_div(static_cast<int64_t>(nb) * token_tiles * 2, 4)));
+    if (xb != nullptr)
+        hipLaunchKernelGGL((fp8_pack_rows_kernel<true>), grid, dim3(256), 0, st, reinterpret_cast<const char*>(xb), out,
+                           m, K, stride * 2, token_tiles, panel_tiles(m, true), nb);
+    else
+        hipLaunchKernelGGL((fp8_pack_rows_kernel<false>), grid, dim3(256), 0, st, reinterpret_cast<const char*>(x), out,
+                           m, K, stride * 4, token_tiles, panel_tiles(m, false), nb);
+    return plm::check_launch("fp8 pack rows");
+}
+
+template <int WR, bool SILU, int MODE, bool SPLIT = false>
+int launch_panel(const PanelArgs& args, hipStream_t st) {
+    PanelArgs a = args;
+    // SILU: whole 128-column blocks of the down phase's activations
+    a.row_tiles = static_cast<int>(SILU ? plm::ceil_div(a.rows, 128) * 128 / (32 * WR) : plm::ceil_div(a.rows, 64 * WR));
+    a.col_tiles = a.x_tiles / kPanelCols;
+    const unsigned grid = static_cast<unsigned>(plm::ceil_div(a.row_tiles, 8) * 8 * a.col_tiles);
+    constexpr int kLds = (MODE == kXPlanes ? 1 : 2) * (4 * WR * 2048 + kPanelCols * kTileBytes);
+    const void* fn = reinterpret_cast<const void*>(&fp8_panel_kernel<WR, SILU, MODE, SPLIT>);
+    int code = plm::allow_large_lds(fn, kLds);
+    if (code != 0) return code;
+    hipLaunchKernelGGL((fp8_panel_kernel<WR, SILU, MODE, SPLIT>), dim3(grid, static_cast<unsigned>(a.splits)),
+                       dim3(256 * WR), kLds, st, a);
+    code = plm::check_launch("fp8 panel kernel");
+    if (code != 0 || !SPLIT) return code;
+    if (SILU) {
+        const int64_t pieces = plm::ceil_div(a.rows, 128) * 16;
+        hipLaunchKernelGGL(fp8_panel_silu_kernel, dim3(static_cast<unsigned>(plm::ceil_div(a.m * pieces, 256))),
+                           dim3(256), 0, st, a.part, a.waves, a.m, a.part_ld, a.rows, a.xout, a.out_tiles, pieces);
+    } else {
+        const int64_t n = a.m * a.rows;
+        hipLaunchKernelGGL(fp8_panel_sum_kernel, dim3(static_cast<unsigned>(plm::ceil_div(n, 256))), dim3(256), 0, st,
+                           a.part, a.waves, n, a.out);
+    }
+    return plm::check_launch("fp8 panel sum");
+}
+
+// Workgroups of 128 weight rows where that leaves one for every compute unit,
+// else of 64, and where those leave many units idle the K slots split over
+// two workgroups a unit: a workgroup alone takes 1.2 us a block whatever the
+// launch, so 7168x16384 at 128 rows goes from 161 us (112 workgroups) to 105,
+// 2048x7168 from 77 to 25; 224 workgroups are better left whole (7168x16384
+// at 256 rows 167 us, split in three 214).
+constexpr int64_t kPanelWhole = 192;   // workgroups from which the slots stay together
+constexpr int64_t kPanelGroups = 512;
+
+int64_t panel_groups(int64_t rows, bool silu, int x_tiles, int wr) {
+    return plm::ceil_div(rows, (silu ? 32 : 64) * wr) * (x_tiles / kPanelCols);
+}
+
+int panel_splits(int64_t rows, bool silu, int x_tiles, int waves) {
+    const int64_t groups = panel_groups(rows, silu, x_tiles, 1);
+    if (groups >= kPanelWhole) return 1;
+    return static_cast<int>(std::min<int64_t>(waves, plm::ceil_div(kPanelGroups, groups)));
+}
+
+// Floats of the slots' sums.
+int64_t panel_part(int64_t rows, bool silu, int x_tiles, int waves, int64_t m) {
+    return panel_splits(rows, silu, x_tiles, waves) == 1 ? 0 : waves * m * rows * (silu ? 2 : 1);
+}
+
+template <bool SILU, int MODE>
+int launch_panel_rows(const PanelArgs& args, float* part, hipStream_t st) {
+    PanelArgs a = args;
+    a.splits = panel_splits(a.rows, SILU, a.x_tiles, a.waves);
+    a.part = part;
+    a.part_ld = a.rows * (SILU ? 2 : 1);
+    if (panel_groups(a.rows, SILU, a.x_tiles, 2) >= plm::cu_count()) return launch_panel<2, SILU, MODE>(a, st);
+    return a.splits == 1 ? launch_panel<1, SILU, MODE>(a, st) : launch_panel<1, SILU, MODE, true>(a, st);
+}
+
+PanelArgs panel_args(const plm::BatchRows& p, const char* x, int x_tiles) {
+    PanelArgs a;
+    std::memset(&a, 0, sizeof(a));
+    for (int i = 0; i < (p.hhi != nullptr ? 2 : 1); ++i) {
+        a.w[i] = p.w[i][0];
+        a.s[i] = p.s[i][0];
+    }
+    a.x = x;
+    a.out = p.out;
+    a.rows = p.rows;
+    a.K = p.K;
+    a.scale_cols = p.scale_cols;
+    a.m = p.m;
+    a.nblocks = static_cast<int>(plm::ceil_div(p.K, 128));
+    a.waves = p.waves;
+    a.x_tiles = x_tiles;
+    a.tiled = p.tiled ? 1 : 0;
+    return a;
+}
+
 template <int TA, int TB, int P, int NWT, bool SILU, int XM, int MAXW>
 int launch(const plm::BatchRows& p, const BatchArgs& args, int chunks, hipStream_t st) {
     BatchArgs a = args;
@@ -450,6 +917,51 @@ int plm::fp8_batch_rows(const BatchRows& p, hipStream_t st) {
                             : launch<2, 2, 1, 1, false, kXF32, 8>(p, a, chunks(2), st);
     return xm == kXBf16 ? launch<2, 4, 1, 1, false, kXBf16, 8>(p, a, chunks(4), st)
                         : launch<2, 2, 1, 1, false, kXF32, 8>(p, a, chunks(2), st);
+}
+
+int plm::fp8_panel_linear(const BatchRows& p, int outs, hipStream_t st) {
+    const bool bf16 = p.xb != nullptr;
+    const int tiles = panel_tiles(p.m, bf16);
+    const int64_t first = panel_bytes(p.m, p.K, bf16);
+    int64_t part = 0;
+    for (int i = 0; i < outs; ++i) part = std::max(part, panel_part(p.out_rows[i], false, tiles, p.waves, p.m));
+    char* x = static_cast<char*>(plm::workspace(static_cast<size_t>(first + part * 4)));
+    if (x == nullptr) return -3;
+    float* sums = reinterpret_cast<float*>(x + first);
+    int code = pack_rows(p.x, p.xb, p.m, p.K, p.x_stride, x, st);
+    for (int i = 0; i < outs && code == 0; ++i) {
+        PanelArgs a = panel_args(p, x, tiles);
+        a.w[0] = p.w[0][i];
+        a.s[0] = p.s[0][i];
+        a.out = p.outs[i];
+        a.rows = p.out_rows[i];
+        code = bf16 ? launch_panel_rows<false, kXBf16>(a, sums, st) : launch_panel_rows<false, kXF32>(a, sums, st);
+    }
+    return code;
+}
+
+int plm::fp8_panel_mlp(const BatchRows& gate_up, const BatchRows& down, hipStream_t st) {
+    const bool bf16 = gate_up.xb != nullptr;
+    const int64_t m = gate_up.m;
+    const int tiles = panel_tiles(m, bf16), out_tiles = panel_tiles(m, false);
+    const int64_t first = panel_bytes(m, gate_up.K, bf16), second = panel_bytes(m, down.K, false);
+    const int64_t part = std::max(panel_part(gate_up.rows, true, tiles, gate_up.waves, m),
+                                  panel_part(down.rows, false, out_tiles, down.waves, m));
+    char* x = static_cast<char*>(plm::workspace(static_cast<size_t>(first + second + part * 4)));
+    if (x == nullptr) return -3;
+    float* sums = reinterpret_cast<float*>(x + first + second);
+    int code = pack_rows(gate_up.x, gate_up.xb, m, gate_up.K, gate_up.x_stride, x, st);
+    if (code != 0) return code;
+    PanelArgs a = panel_args(gate_up, x, tiles);
+    for (int i = 0; i < 2; ++i) {
+        a.w[i] = gate_up.w[i][0];
+        a.s[i] = gate_up.s[i][0];
+    }
+    a.xout = x + first;
+    a.out_tiles = out_tiles;
+    code = bf16 ? launch_panel_rows<true, kXBf16>(a, sums, st) : launch_panel_rows<true, kXF32>(a, sums, st);
+    if (code != 0) return code;
+    return launch_panel_rows<false, kXPlanes>(panel_args(down, x + first, out_tiles), sums, st);
 }
 
 int plm::fp8_batch_pairs(const PairProblem& p, hipStream_t st) {

@@ -1623,28 +1623,11 @@ int zero_page_address(const unsigned char** out) {
     return 0;
 }
 
-// Kernels whose LDS passes 64 KiB must say so once per device: bytes is the
-// most dynamic LDS a launch of fn asks for (its static LDS comes on top).
-int allow_large_lds(const void* fn, int bytes) {
-    static std::mutex mu;
-    static std::vector<std::pair<const void*, int>> done;
-    int dev = 0;
-    hipError_t err = hipGetDevice(&dev);
-    if (err != hipSuccess) return plm::hip_fail(err, "hipGetDevice");
-    std::lock_guard<std::mutex> lock(mu);
-    for (const auto& d : done)
-        if (d.first == fn && d.second == dev) return 0;
-    err = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (err != hipSuccess) return plm::hip_fail(err, "LDS attribute");
-    done.emplace_back(fn, dev);
-    return 0;
-}
-
 template <int TT, int P, bool STAGE, bool FUSED, int MP>
 int launch_down_cfg(const CombineArgs& b, unsigned grid, int nw, size_t shmem, hipStream_t st) {
     const void* fn = reinterpret_cast<const void*>(&fp8_down_kernel<TT, P, STAGE, FUSED, MP>);
     if (shmem > 0) {
-        const int code = allow_large_lds(fn, kDownWaves * kDownStageItems * kDownItemBytes);
+        const int code = plm::allow_large_lds(fn, kDownWaves * kDownStageItems * kDownItemBytes);
         if (code != 0) return code;
     }
     hipLaunchKernelGGL((fp8_down_kernel<TT, P, STAGE, FUSED, MP>), dim3(grid), dim3(nw * plm::kWave), shmem, st, b);
@@ -1745,6 +1728,28 @@ bool rows_fast_ok(const RowsProblem& p) {
 // (fp8_batch.hip), one launch per weight set; the same bits per row.
 int run_rows_batch(const RowsProblem& p, hipStream_t st) {
     const int outs = p.silu ? 1 : p.nwt;  // gate and up share a launch
+    const int n = p.nvar > 0 ? p.nvar : p.nwt;
+    int64_t widest = p.rows;
+    for (int i = 0; i < p.nvar; ++i) widest = std::max(widest, p.vrows[i]);
+    if (!p.silu && p.batch >= plm::panel_from(widest, p.xb != nullptr) && (p.nvar > 0 || p.ngroups == 1)) {
+        // linear, dual and many-linear: one packed copy of the activations
+        plm::BatchRows b;
+        for (int i = 0; i < n; ++i) {
+            b.w[0][i] = p.nvar > 0 ? p.w[0][i] : p.w[i][0];
+            b.s[0][i] = p.nvar > 0 ? p.s[0][i] : p.s[i][0];
+            b.outs[i] = p.nvar > 0 ? p.vout[i] : p.out[i];
+            b.out_rows[i] = p.nvar > 0 ? p.vrows[i] : p.rows;
+        }
+        b.x = p.x;
+        b.xb = p.xb;
+        b.x_stride = p.x_stride;
+        b.K = p.K;
+        b.scale_cols = p.scale_cols;
+        b.m = p.batch;
+        b.waves = rows_waves<false>(plm::ceil_div(p.K, 128));
+        b.tiled = p.tiled;
+        return plm::fp8_panel_linear(b, n, st);
+    }
     for (int i = 0; i < outs; ++i)
         for (int g0 = 0; g0 < p.ngroups; g0 += p.nvar > 0 ? 1 : kMaxGroups) {
             plm::BatchRows b;
@@ -2143,6 +2148,30 @@ int mlp_impl(const uint8_t* gate_weight, const float* gate_scale_inv, const uint
     const uint64_t upp = reinterpret_cast<uintptr_t>(up_weight), usp = reinterpret_cast<uintptr_t>(up_scale_inv);
     const uint64_t dp = reinterpret_cast<uintptr_t>(down_weight), dsp = reinterpret_cast<uintptr_t>(down_scale_inv);
     hipStream_t st = plm::current_stream();
+    const void* x = hidden.f32 != nullptr ? static_cast<const void*>(hidden.f32) : hidden.bf16;
+    if (batch >= plm::panel_from(2 * intermediate_rows, hidden.bf16 != nullptr) && intermediate_rows % 16 == 0 && hidden_cols % 16 == 0 && plm::aligned16(x) &&
+        plm::aligned16(gate_weight) && plm::aligned16(up_weight) && plm::aligned16(down_weight)) {
+        plm::BatchRows gu, dn;
+        gu.w[0][0] = gate_weight;
+        gu.w[1][0] = up_weight;
+        gu.s[0][0] = gate_scale_inv;
+        gu.s[1][0] = up_scale_inv;
+        gu.x = hidden.f32;
+        gu.xb = hidden.bf16;
+        gu.x_stride = gu.K = hidden_cols;
+        gu.rows = dn.K = intermediate_rows;
+        gu.scale_cols = gate_scale_cols;
+        gu.waves = rows_waves<true>(plm::ceil_div(hidden_cols, 128));
+        gu.m = dn.m = batch;
+        dn.w[0][0] = down_weight;
+        dn.s[0][0] = down_scale_inv;
+        dn.out = out;
+        dn.rows = hidden_cols;
+        dn.scale_cols = down_scale_cols;
+        dn.waves = static_cast<int>(
+            std::min<int64_t>(plm::ceil_div(intermediate_rows, 128), plm::kBatchDownWaves));
+        return plm::fp8_panel_mlp(gu, dn, st);
+    }
     float* act = static_cast<float*>(plm::workspace(static_cast<size_t>(batch * intermediate_rows) * sizeof(float)));
     if (act == nullptr) return -3;
     ExpertTables t(&gp, &gsp, &upp, &usp, &dp, &dsp, 1);

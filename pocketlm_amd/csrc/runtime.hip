@@ -187,6 +187,21 @@ int cu_count() {
     return cached[dev];
 }
 
+int allow_large_lds(const void* fn, int bytes) {
+    static std::mutex mu;
+    static std::vector<std::pair<const void*, int>> done;
+    int dev = 0;
+    hipError_t err = hipGetDevice(&dev);
+    if (err != hipSuccess) return hip_fail(err, "hipGetDevice");
+    std::lock_guard<std::mutex> lock(mu);
+    for (const auto& d : done)
+        if (d.first == fn && d.second == dev) return 0;
+    err = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (err != hipSuccess) return hip_fail(err, "LDS attribute");
+    done.emplace_back(fn, dev);
+    return 0;
+}
+
 }  // namespace plm
 
 PLM_EXPORT int pocketlm_set_stream(void* hip_stream) {
