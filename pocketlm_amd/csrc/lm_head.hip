@@ -11,7 +11,7 @@
 //     LDS; a DPP wave sum ends each row.
 //   * topk_level_kernel: slices of 1024 entries, one wave each, keep their
 //     top_k (a larger value first, equal values by the lower row), found by
-//     a bisection on order-preserving keys counted with ballots; levels
+//     a bisection on order-preserving keys; levels
 //     repeat on the survivors until one slice writes the top_k in
 //     descending order (top_k <= 64).  NaN logits rank as -inf.  With fewer
 //     rows than top_k the remaining slots are id -1, logit -inf, the
@@ -93,13 +93,8 @@ __global__ void lm_head_logits_scalar_kernel(const uint16_t* x, const uint16_t* 
     logits[row] = acc;
 }
 
-// Ordering key: NaN as -inf.  a ranks before b when a.v > b.v, or equal
-// values and a lower row.
+// The value a logit ranks by: NaN as -inf.
 __device__ __forceinline__ float key_of(float v) { return v != v ? -__builtin_inff() : v; }
-
-__device__ __forceinline__ bool beats(float va, int64_t ra, float vb, int64_t rb) {
-    return va > vb || (va == vb && ra < rb);
-}
 
 // Order-preserving key of a non-NaN float; 0 marks a missing entry (every
 // float, -inf included, maps above it).
@@ -126,45 +121,95 @@ __device__ __forceinline__ int lanes_below(unsigned long long m) {
 // value first, equal values by position.  The first level's rows rise with
 // the position, and every later level stores a slice's survivors in rank
 // order, slices in row order, so the lower position is the lower row.  No
-// barrier: a 32-step bisection on the order-preserving keys, counted with
-// ballots, finds the top_k-th largest key T; entries above T and the
+// barrier: a bisection on the order-preserving keys finds the top_k-th
+// largest key T (at most 32 steps; what bounds a level is this chain of
+// single-wave steps, about 400 cycles each: 152064 rows, top 50, the levels
+// after the logits 41 -> 24 us with the early end and 64-bit ranks); entries above T and the
 // lowest-placed entries equal to T make exactly top_k survivors (fewer when
 // the slice holds fewer), ranked among themselves.  Missing ranks of a level
 // that is not the last are (NaN, -1), which the next level reads as absent
 // (no kept value is NaN: NaN logits rank as -inf); the last level writes ids
 // + token_offset and logits, (-1, -inf) past the available entries.
 
-// Keys of one slice's entries (0: absent).  FIRST: the values are logits.
-template <bool FIRST, int J>
-__device__ __forceinline__ void slice_keys(float (&val)[J], uint32_t (&key)[J], int64_t avail, int lane) {
+// Keys of one slice's entries (0: absent).  first: the values are logits.
+template <int J>
+__device__ __forceinline__ void slice_keys(bool first, float (&val)[J], uint32_t (&key)[J], int64_t avail, int lane) {
 #pragma unroll
     for (int j = 0; j < J; ++j) {
-        const bool ok = j * 64 + lane < avail && (FIRST || val[j] == val[j]);
-        val[j] = ok ? (FIRST ? key_of(val[j]) : val[j]) : 0.0f;
+        const bool ok = j * 64 + lane < avail && (first || val[j] == val[j]);
+        val[j] = ok ? key_of(val[j]) : 0.0f;
         key[j] = ok ? order_key(val[j]) : 0u;
     }
 }
 
-// The slice's survivors, unranked, in sv / sp [0, kept) (value, position),
-// and entries after them in [kept, 64) that rank after every survivor;
-// returns kept.  Every lane of the wave calls it.
+// Sum, largest and smallest over the wave, by DPP row operations (in every
+// lane, read from lane 63).
+#define PLM_DPP_U32(old, v, ctrl, row_mask) \
+    static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(old), static_cast<int>(v), (ctrl), (row_mask), \
+                                                      0xF, false))
+#define PLM_WAVE_REDUCE(v, op, old)                      \
+    v = op(v, PLM_DPP_U32(old, v, 0xB1, 0xF));           \
+    v = op(v, PLM_DPP_U32(old, v, 0x4E, 0xF));           \
+    v = op(v, PLM_DPP_U32(old, v, 0x141, 0xF));          \
+    v = op(v, PLM_DPP_U32(old, v, 0x140, 0xF));          \
+    v = op(v, PLM_DPP_U32(old, v, 0x142, 0xA));          \
+    v = op(v, PLM_DPP_U32(old, v, 0x143, 0xC));          \
+    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), kSumLane))
+
+__device__ __forceinline__ uint32_t add_u32(uint32_t a, uint32_t b) { return a + b; }
+__device__ __forceinline__ uint32_t max_u32(uint32_t a, uint32_t b) { return a > b ? a : b; }
+__device__ __forceinline__ uint32_t min_u32(uint32_t a, uint32_t b) { return a < b ? a : b; }
+__device__ __forceinline__ uint32_t wave_add(uint32_t v) { PLM_WAVE_REDUCE(v, add_u32, 0u); }
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) { PLM_WAVE_REDUCE(v, max_u32, v); }
+__device__ __forceinline__ uint32_t wave_min(uint32_t v) { PLM_WAVE_REDUCE(v, min_u32, v); }
+
+// A slice's survivors in LDS: value, position, and both as one number that is
+// larger for an earlier rank (0: no survivor).
+struct Survivors {
+    __align__(16) uint64_t order[kMaxTopK];
+    float v[kMaxTopK];
+    int pos[kMaxTopK];
+};
+
+__device__ __forceinline__ uint64_t rank_order(float v, int pos) {
+    // equal values (both zeros) rank by position
+    return static_cast<uint64_t>(order_key(v == 0.0f ? 0.0f : v)) << 32 | (0xFFFFFFFFu - static_cast<uint32_t>(pos));
+}
+
+// The slice's survivors, unranked, in s [0, kept); returns kept.  Every lane
+// of the wave calls it.
 template <int J>
-__device__ __forceinline__ int slice_survivors(const float (&val)[J], const uint32_t (&key)[J], int top_k, float* sv,
-                                               int* sp, int lane) {
+__device__ __forceinline__ int slice_survivors(const float (&val)[J], const uint32_t (&key)[J], int top_k,
+                                               Survivors& s, int lane) {
+    // counted in the lanes, then summed over the wave
     auto count_at_least = [&](uint32_t t) {
-        int c = 0;
+        uint32_t c = 0;
 #pragma unroll
-        for (int j = 0; j < J; ++j) c += __popcll(__ballot(key[j] >= t));
-        return c;
+        for (int j = 0; j < J; ++j) c += key[j] >= t ? 1u : 0u;
+        return static_cast<int>(wave_add(c));
     };
     // T: the largest t with at least top_k entries at or above it (0 when
-    // the slice holds fewer than top_k entries: all of them survive)
-    uint32_t T = 0u;
-    for (int bit = 31; bit >= 0; --bit) {
+    // the slice holds fewer than top_k entries: all of them survive), or any t
+    // with exactly top_k entries at or above it, where the search ends early
+    // (half of the steps on spread-out values).  The 64
+    // lanes' largest keys are 64 >= top_k entries, so T lies between the
+    // smallest and the largest of them and starts with their common bits.
+    uint32_t top = 0u;
+#pragma unroll
+    for (int j = 0; j < J; ++j) top = max_u32(top, key[j]);
+    const uint32_t least = wave_min(top);
+    const uint32_t open = least ^ wave_max(top);
+    const int bits = open == 0u ? 0 : 32 - __builtin_clz(open);  // low bits to find
+    uint32_t T = bits == 32 ? 0u : (least >> bits) << bits;
+    bool exact = false;  // exactly top_k entries at or above T: no ties to choose among
+    for (int bit = bits - 1; bit >= 0 && !exact; --bit) {
         const uint32_t cand = T | (1u << bit);
-        if (count_at_least(cand) >= top_k) T = cand;
+        const int n = count_at_least(cand);
+        if (n >= top_k) T = cand;
+        exact = n == top_k;
     }
-    const int need = top_k - (T == 0u ? 0 : count_at_least(T + 1u));  // ties kept, lowest positions first
+    // ties kept, lowest positions first
+    const int need = exact ? top_k : top_k - (T == 0u ? 0 : count_at_least(T + 1u));
     int ties = 0, kept = 0;
 #pragma unroll
     for (int j = 0; j < J; ++j) {
@@ -175,31 +220,24 @@ __device__ __forceinline__ int slice_survivors(const float (&val)[J], const uint
         const unsigned long long km = __ballot(keep);
         if (keep) {
             const int slot = kept + lanes_below(km);
-            sv[slot] = val[j];
-            sp[slot] = j * 64 + lane;
+            s.v[slot] = val[j];
+            s.pos[slot] = j * 64 + lane;
+            s.order[slot] = rank_order(val[j], j * 64 + lane);
         }
         kept += __popcll(km);  // at most top_k
     }
-    if (lane >= kept) {
-        sv[lane] = -__builtin_inff();
-        sp[lane] = 0x7FFFFFFF;
-    }
+    if (lane >= kept) s.order[lane] = 0;  // after every survivor
     wave_sync();
     return kept;
 }
 
-// Rank of survivor (c, pi) among the 64 slots.
-__device__ __forceinline__ int survivor_rank(const float* sv, const int* sp, float c, int pi) {
+// Rank of survivor i: one 64-bit compare per slot (value and position
+// compares on floats were 6000 of a slice's 19000 cycles).
+__device__ __forceinline__ int survivor_rank(const Survivors& s, int i) {
+    const uint64_t mine = s.order[i];
     int rank = 0;
-#pragma unroll 4
-    for (int j = 0; j < kMaxTopK; j += 4) {
-        const float4 v = *reinterpret_cast<const float4*>(sv + j);
-        const int4 q = *reinterpret_cast<const int4*>(sp + j);
-        rank += (v.x > c) || (v.x == c && q.x < pi);
-        rank += (v.y > c) || (v.y == c && q.y < pi);
-        rank += (v.z > c) || (v.z == c && q.z < pi);
-        rank += (v.w > c) || (v.w == c && q.w < pi);
-    }
+#pragma unroll 16
+    for (int j = 0; j < kMaxTopK; ++j) rank += s.order[j] > mine;
     return rank;
 }
 
@@ -210,8 +248,7 @@ __global__ __launch_bounds__(kTopkWaves * 64) void topk_level_kernel(const float
                                                                      int top_k, float* __restrict__ out_v,
                                                                      int64_t* __restrict__ out_r) {
     constexpr int J = kTopkJ;
-    __shared__ __align__(16) float sv[kTopkWaves][kMaxTopK];
-    __shared__ __align__(16) int sp[kTopkWaves][kMaxTopK];
+    __shared__ Survivors kept_s[kTopkWaves];
     const int wave = static_cast<int>(threadIdx.x >> 6);
     const int lane = static_cast<int>(threadIdx.x & 63);
     const int64_t slice = static_cast<int64_t>(blockIdx.x) * kTopkWaves + wave;
@@ -224,13 +261,13 @@ __global__ __launch_bounds__(kTopkWaves * 64) void topk_level_kernel(const float
 #pragma unroll
     for (int j = 0; j < J; ++j) val[j] = in_v[min(base + j * 64 + lane, n_in - 1)];
     __builtin_amdgcn_sched_barrier(0);  // keep the loads together
-    slice_keys<FIRST, J>(val, key, n_in - base, lane);
-    const int kept = slice_survivors<J>(val, key, top_k, sv[wave], sp[wave], lane);
+    slice_keys<J>(FIRST, val, key, n_in - base, lane);
+    const int kept = slice_survivors<J>(val, key, top_k, kept_s[wave], lane);
     const int64_t o = slice * top_k;
     if (lane < kept) {
-        const float c = sv[wave][lane];
-        const int pi = sp[wave][lane];
-        const int rank = survivor_rank(sv[wave], sp[wave], c, pi);
+        const float c = kept_s[wave].v[lane];
+        const int pi = kept_s[wave].pos[lane];
+        const int rank = survivor_rank(kept_s[wave], lane);
         out_v[o + rank] = c;
         out_r[o + rank] = FIRST ? base + pi : in_r[base + pi];
     } else if (lane < top_k) {
@@ -252,52 +289,57 @@ __global__ __launch_bounds__(kTopkFinalWaves * 64) void topk_final_kernel(const 
                                                                           int64_t token_offset) {
     constexpr int J = kTopkJ;
     static_assert(kTopkFinalWaves * kMaxTopK <= 64 * J, "the survivors of every slice fit one slice");
-    __shared__ __align__(16) float sv[kTopkFinalWaves][kMaxTopK];
-    __shared__ __align__(16) int sp[kTopkFinalWaves][kMaxTopK];
+    __shared__ Survivors kept_s[kTopkFinalWaves];
     __shared__ float cv[kTopkFinalWaves * kMaxTopK];
     __shared__ int64_t cr[kTopkFinalWaves * kMaxTopK];
     const int wave = static_cast<int>(threadIdx.x >> 6);
     const int lane = static_cast<int>(threadIdx.x & 63);
-    const int64_t base = static_cast<int64_t>(wave) * (64 * J);
     const int nslices = static_cast<int>((n_in + 64 * J - 1) / (64 * J));
-    if (base < n_in) {  // whole waves
-        float val[J];
-        uint32_t key[J];
+    // One body for both levels, a loop: its instructions come from memory
+    // once (the logits kernel has streamed a gigabyte through the caches).
+    int64_t base = static_cast<int64_t>(wave) * (64 * J), n = n_in;
+#pragma unroll 1
+    for (int level = 0; level < 2; ++level) {
+        const bool last = level == 1;
+        if (base < n) {  // whole waves
+            float val[J];
+            uint32_t key[J];
+            if (last) {
 #pragma unroll
-        for (int j = 0; j < J; ++j) val[j] = in_v[min(base + j * 64 + lane, n_in - 1)];
-        __builtin_amdgcn_sched_barrier(0);
-        slice_keys<FIRST, J>(val, key, n_in - base, lane);
-        const int kept = slice_survivors<J>(val, key, top_k, sv[wave], sp[wave], lane);
-        const int o = wave * top_k;
-        if (lane < kept) {
-            const float c = sv[wave][lane];
-            const int pi = sp[wave][lane];
-            const int rank = survivor_rank(sv[wave], sp[wave], c, pi);
-            cv[o + rank] = c;
-            cr[o + rank] = FIRST ? base + pi : in_r[base + pi];
-        } else if (lane < top_k) {
-            cv[o + lane] = __builtin_nanf("");
-            cr[o + lane] = -1;
+                for (int j = 0; j < J; ++j) val[j] = cv[min(j * 64 + lane, static_cast<int>(n) - 1)];
+            } else {
+#pragma unroll
+                for (int j = 0; j < J; ++j) val[j] = in_v[min(base + j * 64 + lane, n - 1)];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            slice_keys<J>(FIRST && !last, val, key, n - base, lane);
+            const int kept = slice_survivors<J>(val, key, top_k, kept_s[wave], lane);
+            const int o = wave * top_k;
+            if (lane < kept) {
+                const float c = kept_s[wave].v[lane];
+                const int pi = kept_s[wave].pos[lane];
+                const int rank = survivor_rank(kept_s[wave], lane);
+                if (last) {
+                    out_v[rank] = c;
+                    out_r[rank] = cr[pi] + token_offset;
+                } else {
+                    cv[o + rank] = c;
+                    cr[o + rank] = FIRST ? base + pi : in_r[base + pi];
+                }
+            } else if (lane < top_k) {
+                if (last) {
+                    out_v[lane] = -__builtin_inff();
+                    out_r[lane] = -1;
+                } else {
+                    cv[o + lane] = __builtin_nanf("");
+                    cr[o + lane] = -1;
+                }
+            }
         }
-    }
-    __syncthreads();
-    if (wave != 0) return;
-    const int n2 = nslices * top_k;
-    float val[J];
-    uint32_t key[J];
-#pragma unroll
-    for (int j = 0; j < J; ++j) val[j] = cv[min(j * 64 + lane, n2 - 1)];
-    slice_keys<false, J>(val, key, n2, lane);
-    const int kept = slice_survivors<J>(val, key, top_k, sv[0], sp[0], lane);
-    if (lane < kept) {
-        const float c = sv[0][lane];
-        const int pi = sp[0][lane];
-        const int rank = survivor_rank(sv[0], sp[0], c, pi);
-        out_v[rank] = c;
-        out_r[rank] = cr[pi] + token_offset;
-    } else if (lane < top_k) {
-        out_v[lane] = -__builtin_inff();
-        out_r[lane] = -1;
+        __syncthreads();
+        // the second level: wave 0 over the survivors of every slice
+        n = static_cast<int64_t>(nslices) * top_k;
+        base = wave == 0 ? 0 : n;
     }
 }
 

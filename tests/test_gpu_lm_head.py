@@ -95,3 +95,23 @@ def test_argument_errors(nat):
         nat.lm_head_topk_u16(h.to(torch.bfloat16), w, top_k=2)
     with pytest.raises(ValueError):
         nat.lm_head_topk_u16(h[:8], w, top_k=2)
+
+
+@pytest.mark.parametrize("rows", [3, 64, 65, 1024, 1025, 9000])
+@pytest.mark.parametrize("levels", [1, 2, 40])
+def test_selection_among_few_distinct_logits(nat, rows, levels):
+    """Logits of 1, 2 or 40 distinct values (zeros and negative zeros among
+    them), so that the threshold search ends on ties, between them, or with
+    exactly top_k entries above it: the largest first, equal ones in row order."""
+    g = torch.Generator().manual_seed(rows + levels)
+    value = (torch.randint(0, levels, (rows,), generator=g) - levels // 2).float() * 0.25
+    weight = torch.zeros((rows, 8), dtype=torch.float16)
+    weight[:, 0] = value
+    hidden = torch.zeros((8,), dtype=torch.float16)
+    hidden[0] = 1.0
+    for k in (1, 20, 64):
+        logits, ids = nat.lm_head_topk_u16(hidden.cuda(), weight.cuda(), top_k=k)
+        n = min(k, rows)
+        want = sorted(range(rows), key=lambda r: (-float(value[r]), r))[:n]
+        assert ids[:n].tolist() == want and ids[n:].tolist() == [-1] * (k - n)
+        assert torch.equal(logits[:n].cpu(), value[want])
