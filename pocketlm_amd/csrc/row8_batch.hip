@@ -11,17 +11,16 @@
 // them (row-major activation planes, 64-byte pieces of 16 rows a load, were
 // the bound: gate + up 135 us and down 139 against 112 and 99).
 //
-// A wave takes every activation row (up to 8 token tiles, 256 accumulator
-// registers: one wave per SIMD), so each weight is read once; two token
-// groups sharing the weights through the caches were slower (gate + up 178
-// us).  The KS waves of a workgroup split its K slice and meet in LDS.
+// A workgroup's KS x TG waves: TG groups of token tiles share the weights
+// through the caches, KS parts of the K slice meet in LDS.  One group (a wave
+// with all 8 token tiles, 256 accumulator registers) reads each weight into a
+// compute unit once.
 //
-// What bounds it: bytes in flight.  Two waves per compute unit with two to
-// three 8 KB steps each; four waves were slower (135 us: one workgroup per
-// compute unit then leaves 40 of the 296 row tiles to a second round).
-// Measured at 120 rows of a 3584 / 18944 layer in fp16 (us): q + k + v 30,
-// o 36, gate + up 112 (2.4 TB/s), down 99; the whole layer 13.6 ms one row at
-// a time -> 0.37 ms.
+// What bounds it: loads in flight and their spread.  At 120 rows of a 3584 /
+// 18944 layer in fp16 (us): q + k + v 27, o 25, gate + up 112 (2.4 TB/s),
+// down 94; with one row's activations read again and again gate + up takes 88,
+// with the weights read contiguously as well 77, a bare stream of them 47.
+// The whole layer 13.6 ms one row at a time -> 0.34 ms of kernels.
 #include <algorithm>
 #include <cstring>
 
@@ -59,11 +58,12 @@ __device__ __forceinline__ plm_f32x4 mfma16(plm_u32x4 a, plm_u32x4 b, plm_f32x4 
                                                       __builtin_bit_cast(plm_f16x8, b), c, 0, 0, 0);
 }
 
-template <bool BF16, int TB, int PL, int KS, int P>
-__global__ __launch_bounds__(64 * KS) void row8_batch_kernel(const Row8BatchArgs a) {
-    constexpr int RB = TB < 4 ? TB : 4;  // token tiles per round of the waves' sums
-    __shared__ plm_f32x4 sums[(KS > 1 ? KS / 2 : 1) * 8 * RB * 64];
-    const int ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+template <bool BF16, int TB, int PL, int KS, int P, int TG>
+__global__ __launch_bounds__(64 * KS * TG, TG > 1 ? 2 : 1) void row8_batch_kernel(const Row8BatchArgs a) {
+    constexpr int RB = TB * TG < 4 ? TB : (TG >= 4 ? 1 : 4 / TG);  // token tiles per round of the waves' sums
+    __shared__ plm_f32x4 sums[TG * (KS > 1 ? KS / 2 : 1) * 8 * RB * 64];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tg = wave % TG, ks = wave / TG;
     const int lane = threadIdx.x & 63;
     const int li = lane & 15, qd = lane >> 4;
     const int split = blockIdx.x % a.splits, tile = blockIdx.x / a.splits;
@@ -76,8 +76,8 @@ __global__ __launch_bounds__(64 * KS) void row8_batch_kernel(const Row8BatchArgs
     // blocks past the end read the last one; their results are dropped
     const char* wp = reinterpret_cast<const char*>(mat.packed) + (min(blk0 + li, blocks - 1) * a.K + qd) * 16;
     // the lane's 16 bytes of a step's first token tile; tiles are 1 KB apart
-    const char* xp = reinterpret_cast<const char*>(a.x) + lane * 16;
-    const int64_t plane = a.K / 32 * TB * 1024;
+    const char* xp = reinterpret_cast<const char*>(a.x) + tg * TB * 1024 + lane * 16;
+    const int64_t plane = a.K / 32 * TB * TG * 1024;
     // this wave's 32-column steps: part ks of slice `split` of the row
     const int64_t steps = a.K / 32;
     const int64_t parts = static_cast<int64_t>(a.splits) * KS, part = static_cast<int64_t>(split) * KS + ks;
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(64 * KS) void row8_batch_kernel(const Row8BatchArgs
 #pragma unroll
         for (int pl = 0; pl < PL; ++pl)
 #pragma unroll
-            for (int tb = 0; tb < TB; ++tb) x[slot][pl][tb] = plm_fp8::xload16(xp + pl * plane + (s * TB + tb) * 1024);
+            for (int tb = 0; tb < TB; ++tb) x[slot][pl][tb] = plm_fp8::xload16(xp + pl * plane + (s * TB * TG + tb) * 1024);
     };
     auto compute = [&](int slot, int) {
 #pragma unroll
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(64 * KS) void row8_batch_kernel(const Row8BatchArgs
                 for (int t = 0; t < 8; ++t)
 #pragma unroll
                     for (int tb = 0; tb < RB; ++tb)
-                        sums[(((ks - half) * 8 + t) * RB + tb) * 64 + lane] = acc[t][r + tb];
+                        sums[(((tg * half + ks - half) * 8 + t) * RB + tb) * 64 + lane] = acc[t][r + tb];
             }
             __syncthreads();
             if (ks < half) {
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(64 * KS) void row8_batch_kernel(const Row8BatchArgs
                 for (int t = 0; t < 8; ++t)
 #pragma unroll
                     for (int tb = 0; tb < RB; ++tb)
-                        acc[t][r + tb] = acc[t][r + tb] + sums[((ks * 8 + t) * RB + tb) * 64 + lane];
+                        acc[t][r + tb] = acc[t][r + tb] + sums[(((tg * half + ks) * 8 + t) * RB + tb) * 64 + lane];
             }
             __syncthreads();
         }
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(64 * KS) void row8_batch_kernel(const Row8BatchArgs
     if (ks != 0) return;
 #pragma unroll
     for (int tb = 0; tb < TB; ++tb) {
-        const int m = 16 * tb + li;
+        const int m = 16 * (tg * TB + tb) + li;
         if (m >= a.m) continue;
         const float f = a.inv != nullptr ? a.inv[m] : 1.0f;
         float* o = a.part + (static_cast<int64_t>(split) * a.m + m) * a.ld + mat.out_col;
@@ -166,23 +166,32 @@ __global__ __launch_bounds__(64 * KS) void row8_batch_kernel(const Row8BatchArgs
     }
 }
 
-template <bool BF16, int TB, int PL, int KS, int P>
+template <bool BF16, int TB, int PL, int KS, int P, int TG = 1>
 int launch(const Row8BatchArgs& a, hipStream_t st) {
-    hipLaunchKernelGGL((row8_batch_kernel<BF16, TB, PL, KS, P>), dim3(static_cast<unsigned>(a.tiles * a.splits)),
-                       dim3(64 * KS), 0, st, a);
+    hipLaunchKernelGGL((row8_batch_kernel<BF16, TB, PL, KS, P, TG>), dim3(static_cast<unsigned>(a.tiles * a.splits)),
+                       dim3(64 * KS * TG), 0, st, a);
     return plm::check_launch("row8 batch kernel");
 }
 
-// Steps in flight (P) and waves that split a slice (KS) by token tiles: what
-// fits the registers (8 tiles: 256 accumulators + 3 x 64; two or three planes
-// leave 2 steps).
+// Steps in flight (P), waves that split a slice (KS) and token groups (TG) by
+// token tiles.  One plane, 8 tiles: one wave holds them all (256 accumulators
+// + 3 x 64) where the weight rows alone fill the compute units; with K slices
+// two groups of 4 tiles put two waves on a SIMD (q + k + v 30 -> 27 us, gate +
+// up 112 -> 142).  Several planes: groups of 2 tiles, with two planes 3 steps in flight (o 36
+// -> 25 us, down 99 -> 94).
 template <bool BF16, int PL>
 int launch_m(const Row8BatchArgs& a, hipStream_t st) {
-    switch (plm::row8_token_tiles(a.m)) {
-        case 1: return launch<BF16, 1, PL, 4, 3>(a, st);
-        case 2: return launch<BF16, 2, PL, 4, 3>(a, st);
-        case 4: return launch<BF16, 4, PL, 2, 2>(a, st);
-        default: return launch<BF16, 8, PL, 2, PL == 1 ? 3 : 2>(a, st);
+    const int tiles = plm::row8_token_tiles(a.m);
+    if (tiles == 1) return launch<BF16, 1, PL, 4, 3>(a, st);
+    if (tiles == 2) return launch<BF16, 2, PL, 4, 3>(a, st);
+    if constexpr (PL == 1) {
+        if (tiles == 4) return launch<BF16, 4, PL, 2, 2>(a, st);
+        if (a.splits > 1) return launch<BF16, 4, PL, 2, 2, 2>(a, st);
+        return launch<BF16, 8, PL, 2, 3>(a, st);
+    } else {
+        constexpr int P = PL == 2 ? 3 : 2;  // three planes of three steps do not fit the registers
+        if (tiles == 4) return launch<BF16, 2, PL, 2, P, 2>(a, st);
+        return launch<BF16, 2, PL, 1, P, 4>(a, st);
     }
 }
 
