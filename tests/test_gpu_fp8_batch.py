@@ -109,3 +109,31 @@ def test_pairs_vs_the_oracle(nat, oracle_mod, experts, batch, inter, hid, top, d
            for a, v in zip(args, ([experts, -1, 0], [0, 0, batch], [1.0, 1.0, 1.0]))]
     out, n = nat.fp8_e4m3_block_mlp_many_pair_weighted_nosync(items, x, *bad)
     assert int(n.item()) == 3 and torch.equal(out, got)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_other_entry_points_have_the_bits_of_one_row_calls(nat, dtype):
+    """Weights of several sizes in one call, 8-row tiles, and the many-expert
+    MLPs (66 experts: two tables of addresses), below and above the panel
+    kernel's row counts."""
+    weights = [_fp8(rows, 400, rows) for rows in (24, 136, 300)]
+    packed = [nat.pack_fp8_tiles8(w) for w, _s in weights]
+    items = [(*_fp8(48, 144, 3 * e), *_fp8(48, 144, 3 * e + 1), *_fp8(144, 48, 3 * e + 2)) for e in range(66)]
+    route = torch.rand((66, 150), generator=torch.Generator().manual_seed(1)).cuda()
+    for m in (9, 20, 40, 150):
+        print("entry points", m, dtype, flush=True)
+        x = _x(m, 400, m, dtype)
+        for (w, s), p, y in zip(weights, packed, nat.fp8_e4m3_block_linear_many_f32(weights, x)):
+            want = nat.fp8_e4m3_block_linear_f32(w, s, x)
+            assert torch.equal(y, want)
+            assert torch.equal(nat.fp8_e4m3_block_linear_tiles8_f32(p, s, x), want)
+            assert torch.equal(want[m - 1:], nat.fp8_e4m3_block_linear_f32(w, s, x[m - 1:]))
+        h = _x(m, 144, m + 1, dtype)
+        many = nat.fp8_e4m3_block_mlp_many_f32(items, h)
+        for e in (0, 1, 63, 64, 65):
+            assert torch.equal(many[e], nat.fp8_e4m3_block_mlp_f32(*items[e], h)), e
+        r = route[:, :m].contiguous()
+        rows = nat.fp8_e4m3_block_mlp_many_row_weighted_f32(items, h, r)
+        for i in (0, 8, m - 1):
+            one = nat.fp8_e4m3_block_mlp_many_row_weighted_f32(items, h[i:i + 1], r[:, i:i + 1].contiguous())
+            assert torch.equal(rows[i:i + 1], one), i
