@@ -491,7 +491,7 @@ __device__ __forceinline__ plm_u32x4 quad_part(plm_u32x4 v) {
 // same piece, so each loads one 16-byte part of it and the parts are
 // exchanged across the quad, one load instruction per block instead of two
 // (bf16) or four (fp32).  o 7168x16384 at one row: 26.2 -> 23.0 us (bf16),
-// 36.2 -> 28.9 us (fp32).  The gate/up burst loop loads on the live lanes
+// 36.2 -> 28.9 us (fp32; 24.3 with quad_operands).  The gate/up burst loop loads on the live lanes
 // only and gains nothing from it.
 template <bool XB>
 __device__ __forceinline__ plm_u32x4 load_xpart(const char* piece, int lane) {
@@ -536,14 +536,30 @@ __device__ __forceinline__ XPiece<XB> pair_piece(const XPiece<XB>& own, int lane
 
 template <bool XB>
 __device__ __forceinline__ XPiece<XB> quad_piece(plm_u32x4 part) {
+    static_assert(XB, "fp32 parts are split before the exchange (quad_operands)");
     XPiece<XB> x;
     x.v[0] = quad_part<0>(part);
     x.v[1] = quad_part<1>(part);
-    if constexpr (!XB) {
-        x.v[2] = quad_part<2>(part);
-        x.v[3] = quad_part<3>(part);
-    }
     return x;
+}
+
+// The B operands of fp32 parts: each lane splits its own four values into hi
+// and lo and the halves are exchanged, a quarter of the conversions of
+// exchanging first (they are the same in the quad's four lanes).
+// o 7168x16384 at one row 27.6 -> 24.3 us, q_b 24576x1536 12.85 -> 12.55.
+template <bool SAN>
+__device__ __forceinline__ BOperands<false, SAN> quad_operands(plm_u32x4 part) {
+    plm_bf16x8 h, l;
+    split8<SAN>(part, part, h, l);
+    const plm_u32x4 hv = __builtin_bit_cast(plm_u32x4, h), lv = __builtin_bit_cast(plm_u32x4, l);
+    const plm_u32x4 hl = {hv.x, hv.y, lv.x, lv.y};
+    const plm_u32x4 p0 = quad_part<0>(hl), p1 = quad_part<1>(hl), p2 = quad_part<2>(hl), p3 = quad_part<3>(hl);
+    BOperands<false, SAN> b;
+    b.h0 = __builtin_bit_cast(plm_bf16x8, plm_u32x4{p0.x, p0.y, p1.x, p1.y});
+    b.h1 = __builtin_bit_cast(plm_bf16x8, plm_u32x4{p2.x, p2.y, p3.x, p3.y});
+    b.l0 = __builtin_bit_cast(plm_bf16x8, plm_u32x4{p0.z, p0.w, p1.z, p1.w});
+    b.l1 = __builtin_bit_cast(plm_bf16x8, plm_u32x4{p2.z, p2.w, p3.z, p3.w});
+    return b;
 }
 
 template <int TT, int U, int NWT, bool XB, bool SAN>
@@ -629,26 +645,35 @@ __device__ __forceinline__ void rows_pass(const RowsArgs& a, const uint8_t* cons
             float sc[NWT];
 #pragma unroll
             for (int n = 0; n < NWT; ++n) sc[n] = lane_value(sv[n], k);
-            XPiece<XB> xv;
-            if constexpr (XS == 1) {
-                xv = quad_piece<XB>(x[slot].v[0]);
-            } else if constexpr (XS == 2) {
-                xv = pair_piece<XB>(x[slot], lane);
-            } else {
-                xv = x[slot];
-            }
+            // the row's last block: columns past K add nothing
+            const bool in =
+                !ragged || (wave + static_cast<int64_t>(kb + k) * nw) * 128 + lane_col < K;
             plm_u32x4 qv[NT];
 #pragma unroll
-            for (int t = 0; t < NT; ++t) qv[t] = q[slot][t];
-            if (ragged) {
-                // the row's last block: columns past K add nothing
-                const bool in = (wave + static_cast<int64_t>(kb + k) * nw) * 128 + lane_col < K;
-#pragma unroll
-                for (int t = 0; t < NT; ++t) qv[t] = in ? qv[t] : plm_u32x4{0, 0, 0, 0};
-#pragma unroll
-                for (int i = 0; i < (XB ? 2 : 4); ++i) xv.v[i] = in ? xv.v[i] : plm_u32x4{0, 0, 0, 0};
+            for (int t = 0; t < NT; ++t) {
+                qv[t] = q[slot][t];
+                if (ragged) qv[t] = in ? qv[t] : plm_u32x4{0, 0, 0, 0};
             }
-            const BOperands<XB, SAN> bo(xv);
+            BOperands<XB, SAN> bo;
+            if constexpr (XS == 1 && !XB) {
+                plm_u32x4 part = x[slot].v[0];
+                if (ragged) part = in ? part : plm_u32x4{0, 0, 0, 0};
+                bo = quad_operands<SAN>(part);
+            } else {
+                XPiece<XB> xv;
+                if constexpr (XS == 1) {
+                    xv = quad_piece<XB>(x[slot].v[0]);
+                } else if constexpr (XS == 2) {
+                    xv = pair_piece<XB>(x[slot], lane);
+                } else {
+                    xv = x[slot];
+                }
+                if (ragged) {
+#pragma unroll
+                    for (int i = 0; i < (XB ? 2 : 4); ++i) xv.v[i] = in ? xv.v[i] : plm_u32x4{0, 0, 0, 0};
+                }
+                bo = BOperands<XB, SAN>(xv);
+            }
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
                 const plm_f32x4 d = tile_block<XB, SAN>(qv[t], bo);

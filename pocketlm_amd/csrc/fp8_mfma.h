@@ -110,6 +110,7 @@ __device__ __forceinline__ XPiece<XB> load_xpiece(const void* p, bool live) {
 template <bool XB, bool SAN>
 struct BOperands {
     plm_bf16x8 h0, h1, l0, l1;
+    BOperands() = default;
     __device__ __forceinline__ explicit BOperands(const XPiece<XB>& x) {
         if constexpr (XB) {
             h0 = __builtin_bit_cast(plm_bf16x8, x.v[0]);
