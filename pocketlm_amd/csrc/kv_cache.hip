@@ -777,7 +777,7 @@ __global__ __launch_bounds__(kNormThreads) void post_attention_kernel(const uint
 // A prompt through the layer takes up to kRow8BatchRows rows at a time
 // through each step, so that every weight is read once for all of them
 // (120 rows one at a time: 120 times; 3584 / 18944 in fp16, 120 rows: 13.6 ->
-// 0.37 ms).  The projections run on the matrix
+// 0.40 ms a call).  The projections run on the matrix
 // cores (row8_batch.hip) and leave sums per K slice, which the next kernel
 // adds; activations go to them as planes of 16-bit values in the order
 // row8.h describes.  The values that a row's step rounds to the
@@ -1299,7 +1299,8 @@ int commit_rows(KvSession* s, int64_t count) {
 
 // A prompt: every row through the layer, then committed.  Prompts of up to
 // kPromptDecodeRows rows go one row at a time, so that they have the bits of
-// decode steps (a verifier's draft; 8 rows 0.9 ms, 9 rows together 0.2 ms);
+// decode steps (a verifier's draft; 3584 / 18944: 8 rows 954 us a call, 9
+// rows together 256, 64 rows 319, 120 rows 393);
 // longer ones kRow8BatchRows at a time where the shape suits
 // the row kernels (whole 32-column steps, 16-byte K pieces).
 constexpr int64_t kPromptDecodeRows = 8;
