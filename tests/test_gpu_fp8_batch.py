@@ -137,3 +137,32 @@ def test_other_entry_points_have_the_bits_of_one_row_calls(nat, dtype):
         for i in (0, 8, m - 1):
             one = nat.fp8_e4m3_block_mlp_many_row_weighted_f32(items, h[i:i + 1], r[:, i:i + 1].contiguous())
             assert torch.equal(rows[i:i + 1], one), i
+
+
+def test_prompt_calls_captured_cold(nat):
+    """The first panel-kernel calls on a stream, made under capture (scratch
+    and the large-LDS setting included): every replay, with eager work in
+    between, equals the eager call."""
+    w, s = _fp8(328, 1040, 5)
+    mlp = [*_fp8(272, 1040, 6), *_fp8(272, 1040, 7), *_fp8(1040, 272, 8)]
+    items = [(*_fp8(144, 1040, 3 * e), *_fp8(144, 1040, 3 * e + 1), *_fp8(1040, 144, 3 * e + 2)) for e in range(5)]
+    x = _x(70, 1040, 9, torch.float32)
+    pi = torch.arange(140, device="cuda") % 5
+    pr = torch.arange(140, device="cuda") // 2
+    pw = torch.rand(140, generator=torch.Generator().manual_seed(2)).cuda()
+
+    def step():
+        return (nat.fp8_e4m3_block_linear_f32(w, s, x), nat.fp8_e4m3_block_mlp_f32(*mlp, x),
+                *nat.fp8_e4m3_block_mlp_many_pair_weighted_nosync(items, x, pi, pr, pw))
+
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step()
+    for trial in range(3):
+        x.copy_(_x(70, 1040, 20 + trial, torch.float32))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [t.clone() for t in captured]
+        for a, b in zip(got, step()):
+            assert torch.equal(a, b), trial
