@@ -784,6 +784,7 @@ __global__ __launch_bounds__(kNormThreads) void post_attention_kernel(const uint
 // storage type are rounded the same here; sums run in another order.
 
 constexpr int kRowThreads = 1024;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Stores eight columns of row `row`, its piece (g, q) at 4 g + q, into a
 // plane of `tiles` token tiles (row8.h).
@@ -808,31 +809,38 @@ __device__ __forceinline__ uint32_t block_max(uint32_t v, uint32_t* red) {
     return v;
 }
 
-// fp32 value -> its 16-bit parts, whose sum times `scale`'s inverse is the
-// value to 2^-24 of it (fp16: two parts rounded to nearest, the row scaled by
-// a power of two that puts its largest value at 2^14..2^15, so a part below
-// fp16's range is below 2^-40 of the row's largest value) or exactly (bf16:
-// three parts of 8 bits).  Infinities and NaNs stay whole in the first part.
+// The leading 8 significant bits of a finite value.
+__device__ __forceinline__ float lead8(float v) { return __uint_as_float(__float_as_uint(v) & 0xFFFF0000u); }
+
+// fp32 value -> three 16-bit parts of 8 significant bits each, whose sum is
+// the value times `scale`: exactly in bf16 (scale 1), and in fp16 for values
+// from 2^-15 of the row's largest up (smaller ones to 2^-39 of the largest:
+// the row is scaled by a power of two that puts its largest value at
+// 2^14..2^15).  8 bits and not fp16's 11: a matrix instruction keeps more of
+// short products (o 1.05e-7 -> 1.01e-7 off 64 bits).  Infinities and NaNs stay
+// whole in the first part.
 template <bool BF16>
-__device__ __forceinline__ void split_parts(float v, float scale, uint32_t (&p)[3]) {
-    if constexpr (BF16) {
-        const uint32_t b = __float_as_uint(v);
-        if ((b & 0x7F800000u) == 0x7F800000u) {
-            p[0] = (b & 0x007FFFFFu) != 0 ? 0x7FC0u : b >> 16;
-            p[1] = p[2] = 0;
-            return;
+__device__ __forceinline__ void split_parts(float v, float scale, uint32_t (&p)[plm::kRow8Parts]) {
+    const float s = v * scale;
+    const uint32_t b = __float_as_uint(s);
+    if ((b & 0x7F800000u) == 0x7F800000u) {
+        const uint32_t inf = (BF16 ? 0x7F80u : 0x7C00u) | (b >> 16 & 0x8000u);
+        p[0] = (b & 0x007FFFFFu) != 0 ? (BF16 ? 0x7FC0u : 0x7E00u) : inf;
+        p[1] = p[2] = 0;
+        return;
+    }
+    float r = s;
+#pragma unroll
+    for (int k = 0; k < plm::kRow8Parts; ++k) {
+        const float h = k < 2 ? lead8(r) : r;
+        if constexpr (BF16) {
+            p[k] = __float_as_uint(h) >> 16;
+            r -= lead8(h);
+        } else {
+            const _Float16 part = static_cast<_Float16>(h);
+            p[k] = __builtin_bit_cast(uint16_t, part);
+            r -= static_cast<float>(part);
         }
-        p[0] = b >> 16;
-        const float r1 = v - __uint_as_float(b & 0xFFFF0000u);
-        p[1] = __float_as_uint(r1) >> 16;
-        const float r2 = r1 - __uint_as_float(__float_as_uint(r1) & 0xFFFF0000u);
-        p[2] = __float_as_uint(r2) >> 16;
-    } else {
-        const float s = v * scale;
-        const _Float16 h = static_cast<_Float16>(s);
-        const float r = s - static_cast<float>(h);
-        p[0] = __builtin_bit_cast(uint16_t, h);
-        p[1] = r - r == 0.0f ? __builtin_bit_cast(uint16_t, static_cast<_Float16>(r)) : 0;
     }
 }
 
@@ -844,20 +852,31 @@ __device__ __forceinline__ float row_scale(uint32_t max_bits, float& inverse) {
     return __uint_as_float((268u - e) << 23);
 }
 
-// storage(rms_norm(hidden) * w) of each row, in pieces.
+// storage(rms_norm(hidden) * w) of each row, in pieces.  The row's squares are
+// summed as the decode step's q/k/v launch sums them, so that the values have
+// its bits: a scale one bit off turns the 16-bit rounding of some of them, and
+// those show in k and v.
+constexpr int kNormRowThreads = 64 * plm::kRow8Waves;
+
 template <bool BF16>
-__global__ __launch_bounds__(kRowThreads) void norm_rows_kernel(const uint16_t* __restrict__ hidden,
-                                                                const uint16_t* __restrict__ w,
-                                                                uint16_t* __restrict__ x, int tiles, int64_t n, float eps) {
+__global__ __launch_bounds__(kNormRowThreads) void norm_rows_kernel(const uint16_t* __restrict__ hidden,
+                                                                    const uint16_t* __restrict__ w,
+                                                                    uint16_t* __restrict__ x, int tiles, int64_t n,
+                                                                    float eps) {
 #pragma clang fp contract(off)
-    __shared__ float red[kRowThreads / 64];
+    __shared__ float red[plm::kRow8Waves];
     const uint16_t* h = hidden + blockIdx.x * n;
     float s = 0.0f;
     for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
         const float v = rd16(h[i], BF16);
         s += v * v;
     }
-    const float scale = 1.0f / sqrtf(block_sum(s, red) / static_cast<float>(n) + eps);
+    s = plm_wave_sum(s);
+    if ((threadIdx.x & 63) == kSumLane) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    s = 0.0f;
+    for (int i = 0; i < static_cast<int>(blockDim.x >> 6); ++i) s += red[i];
+    const float scale = 1.0f / sqrtf(s / static_cast<float>(n) + eps);
     for (int64_t p = threadIdx.x; p < n / 8; p += blockDim.x) {
         uint32_t v[8];
 #pragma unroll
@@ -869,10 +888,17 @@ __global__ __launch_bounds__(kRowThreads) void norm_rows_kernel(const uint16_t* 
     }
 }
 
-// Sum over the K slices of a projection's element.
-__device__ __forceinline__ float sum_slices(const float* part, int64_t at, int splits, int64_t stride) {
-    float v = part[at];
-    for (int s = 1; s < splits; ++s) v += part[at + s * stride];
+// Sum over the K slices (a power of two) of a projection's elements (a float,
+// or four), in groups of four: their loads are in flight together and the sum
+// is closer to 64 bits than a chain of sixteen adds.
+template <class T>
+__device__ __forceinline__ T sum_slices(const float* part, int64_t at, int splits, int64_t stride) {
+    const float* p = part + at;
+    auto slice = [&](int s) { return *reinterpret_cast<const T*>(p + s * stride); };
+    if (splits == 1) return slice(0);
+    if (splits == 2) return slice(0) + slice(1);
+    T v = (slice(0) + slice(1)) + (slice(2) + slice(3));
+    for (int s = 4; s < splits; s += 4) v = v + ((slice(s) + slice(s + 1)) + (slice(s + 2) + slice(s + 3)));
     return v;
 }
 
@@ -896,12 +922,12 @@ __global__ __launch_bounds__(64) void qk_rope_rows_kernel(const float* __restric
     const int64_t H = static_cast<int64_t>(nh) * hd, kvw = static_cast<int64_t>(nkv) * hd;
     const uint16_t* bias = is_q ? q_bias : k_bias;
     for (int d = lane; d < hd; d += 64)
-        src[d] = sum_slices(part, row * ld + (is_q ? 0 : H) + at + d, splits, stride) +
+        src[d] = sum_slices<float>(part, row * ld + (is_q ? 0 : H) + at + d, splits, stride) +
                  (bias != nullptr ? rd16(bias[at + d], BF16) : 0.0f);
     if (!is_q)
         for (int d = lane; d < hd; d += 64)
             v_rows[row * kvw + at + d] =
-                wr16(sum_slices(part, row * ld + H + kvw + at + d, splits, stride) +
+                wr16(sum_slices<float>(part, row * ld + H + kvw + at + d, splits, stride) +
                          (v_bias != nullptr ? rd16(v_bias[at + d], BF16) : 0.0f),
                      BF16);
     __syncthreads();
@@ -922,13 +948,19 @@ __global__ __launch_bounds__(kRowThreads) void split_rows_kernel(const float* __
     float scale = 1.0f;
     if (SILU || !BF16) {
         uint32_t top = 0;
-        for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
+        for (int64_t i = 4 * threadIdx.x; i < n; i += 4 * blockDim.x) {  // n is a multiple of 32
+            f32x4* at = reinterpret_cast<f32x4*>(v + i);
             if constexpr (SILU) {
-                const float g = sum_slices(part, row * ld + i, splits, rows * ld);
-                const float u = sum_slices(part, row * ld + n + i, splits, rows * ld);
-                v[i] = (g / (1.0f + expf(-g))) * u;
+                const f32x4 g = sum_slices<f32x4>(part, row * ld + i, splits, rows * ld);
+                const f32x4 u = sum_slices<f32x4>(part, row * ld + n + i, splits, rows * ld);
+                f32x4 a;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) a[j] = (g[j] / (1.0f + expf(-g[j]))) * u[j];
+                *at = a;
             }
-            top = max(top, __float_as_uint(v[i]) & 0x7FFFFFFFu);
+            const f32x4 a = *at;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) top = max(top, __float_as_uint(a[j]) & 0x7FFFFFFFu);
         }
         top = block_max(top, red);  // also orders the row's values before the pass below
         if constexpr (!BF16) {
@@ -937,12 +969,12 @@ __global__ __launch_bounds__(kRowThreads) void split_rows_kernel(const float* __
             if (threadIdx.x == 0) inv[row] = inverse;
         }
     }
-    constexpr int PL = plm::row8_planes(BF16);
+    constexpr int PL = plm::kRow8Parts;
     for (int64_t p = threadIdx.x; p < n / 8; p += blockDim.x) {
         uint32_t o[PL][8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            uint32_t t[3];
+            uint32_t t[PL];
             split_parts<BF16>(v[piece_column(p, j)], scale, t);
 #pragma unroll
             for (int k = 0; k < PL; ++k) o[k][j] = t[k];
@@ -965,7 +997,7 @@ __global__ __launch_bounds__(kRowThreads) void post_attention_rows_kernel(const 
     const int64_t at = blockIdx.x * n, stride = gridDim.x * n;
     float s = 0.0f;
     for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-        const float r = rd16(hidden[at + i], BF16) + rd16(wr16(sum_slices(part, at + i, splits, stride), BF16), BF16);
+        const float r = rd16(hidden[at + i], BF16) + rd16(wr16(sum_slices<float>(part, at + i, splits, stride), BF16), BF16);
         resid[at + i] = r;
         const float rq = rd16(wr16(r, BF16), BF16);
         s += rq * rq;
@@ -987,7 +1019,7 @@ template <bool BF16>
 __global__ __launch_bounds__(256) void add_rows_kernel(const float* __restrict__ resid, const float* __restrict__ part,
                                                        int splits, uint16_t* __restrict__ out, int64_t n) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (i < n) out[i] = wr16(resid[i] + sum_slices(part, i, splits, n), BF16);
+    if (i < n) out[i] = wr16(resid[i] + sum_slices<float>(part, i, splits, n), BF16);
 }
 
 struct LayerLengths {
@@ -1188,7 +1220,7 @@ int dense_prompt_rows(KvSession* s, int64_t layer, const DenseArgs& a, int m) {
     if (nsplit > kMaxSplits) return plm::fail(106, "context too long for one attention launch");
     const int64_t row_part = a.nh * nsplit * hd * 4;
     const int64_t arows = std::max<int64_t>(1, std::min<int64_t>(m, kPromptPartBytes / row_part));
-    constexpr int PL = plm::row8_planes(BF16);
+    constexpr int PL = plm::kRow8Parts;
     const int64_t qkv_ld = H + 2 * kvw;
     const int s_qkv = plm::row8_batch_splits(qkv_ld, H), s_o = plm::row8_batch_splits(H, H);
     const int s_gu = plm::row8_batch_splits(2 * I, H), s_down = plm::row8_batch_splits(H, I);
@@ -1236,7 +1268,9 @@ int dense_prompt_rows(KvSession* s, int64_t layer, const DenseArgs& a, int m) {
         return plm::row8_batch(b, stream);
     };
 
-    hipLaunchKernelGGL((norm_rows_kernel<BF16>), per_row, row_block, 0, stream, a.hidden, a.input_norm, x, tiles, H, a.eps);
+    const dim3 norm_block(static_cast<unsigned>(64 * std::min<int64_t>(plm::ceil_div(H, 64), plm::kRow8Waves)));
+    hipLaunchKernelGGL((norm_rows_kernel<BF16>), per_row, norm_block, 0, stream, a.hidden, a.input_norm, x, tiles, H,
+                       a.eps);
     if ((code = plm::check_launch("input norm rows")) != 0) return code;
     code = project({{a.q_w, H, 0}, {a.k_w, kvw, H}, {a.v_w, kvw, H + kvw}}, H, qkv_ld, 1, s_qkv);
     if (code != 0) return code;

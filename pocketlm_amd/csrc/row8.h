@@ -41,17 +41,20 @@ int row8_gemv(const uint16_t* hidden, const float* hidden_f32, const Row8Mat* ma
               hipStream_t st);
 int row8_gemv_x(const Row8X& x, const Row8Mat* mats, int n, int64_t K, int dtype_code, hipStream_t st);
 
+// Waves of a GEMV workgroup over K columns: min(K / 64 rounded up, kRow8Waves).
+constexpr int kRow8Waves = 8;
+
 // ------------------------------------------------------------------ many rows (row8_batch.hip)
 //
 // Up to kRow8BatchRows activation rows against row8 weights on the matrix
 // cores.  The activations come as planes of storage-type values whose sum is
-// the row (one plane for fp16 / bf16 rows; fp32 rows as row8_planes parts),
+// the row (one plane for fp16 / bf16 rows; fp32 rows as kRow8Parts parts),
 // in the order the lanes of the kernel read them: 16-byte pieces
 // [K / 32][token tile][q = 0..3][token of the tile], piece (g, q) of a row
 // being its columns 32 g + 4 j + q, j = 0..7 (one load of a lane's weights
 // holds one column of its 8 rows).
 constexpr int kRow8BatchRows = 128;
-constexpr int row8_planes(bool bf16) { return bf16 ? 3 : 2; }
+constexpr int kRow8Parts = 3;
 // 16-row token tiles of an activation plane (rows past m may hold anything).
 constexpr int row8_token_tiles(int64_t m) { return m <= 16 ? 1 : (m <= 32 ? 2 : (m <= 64 ? 4 : 8)); }
 constexpr int64_t row8_plane_bytes(int64_t m, int64_t K) { return K / 32 * row8_token_tiles(m) * 1024; }

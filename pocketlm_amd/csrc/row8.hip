@@ -14,7 +14,7 @@
 
 namespace {
 
-constexpr int kMaxWaves = 8;
+constexpr int kMaxWaves = plm::kRow8Waves;
 constexpr int kUnroll = 8;       // chunks whose loads are issued together
 constexpr int kMaxMats = plm::kRow8MaxMats;  // matrices per fused launch
 using plm::Row8Mat;
