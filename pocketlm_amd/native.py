@@ -1766,12 +1766,15 @@ class NativeKvSession:
         _check("kv_dense_layer_decode_u16_ext_packed_rows8", code)
         return out
 
-    def _dense_layer_args(self, hidden, rows, input_norm_weight, post_norm_weight, *packed, hidden_size,
-                          intermediate_size, num_heads, num_kv_heads, head_dim=None, rms_eps, rope_theta, q_bias=None,
-                          k_bias=None, v_bias=None, q_norm_weight=None, k_norm_weight=None):
+    def _dense_layer_args(self, hidden, rows, input_norm_weight, post_norm_weight, q_weight_packed, k_weight_packed,
+                          v_weight_packed, o_weight_packed, gate_weight_packed, up_weight_packed, down_weight_packed,
+                          *, hidden_size, intermediate_size, num_heads, num_kv_heads, head_dim=None, rms_eps,
+                          rope_theta, q_bias=None, k_bias=None, v_bias=None, q_norm_weight=None, k_norm_weight=None):
         """The checks of a dense layer call: (hidden on the session's device,
         the other tensors in the C ABI's order, the sizes and constants)."""
         raw = [hidden, input_norm_weight, post_norm_weight]
+        packed = [q_weight_packed, k_weight_packed, v_weight_packed, o_weight_packed, gate_weight_packed,
+                  up_weight_packed, down_weight_packed]
         if any(t.dtype != self.dtype for t in raw):
             raise TypeError(f"dense_layer_decode_packed_rows8 requires {self.dtype} raw tensors")
         if any(t.dtype != torch.uint16 for t in packed):
@@ -1805,7 +1808,8 @@ class NativeKvSession:
     def dense_layer_prefill_packed_rows8(self, layer: int, hidden: torch.Tensor, *weights: torch.Tensor,
                                          **kwargs) -> torch.Tensor:
         """kv_dense_layer_prefill_u16_ext's loop (fp16_kv_cache.cpp:1591-1673)
-        over the packed weights: every row decoded, then committed.  Up to 8
+        over the packed weights, taken as dense_layer_decode_packed_rows8 takes
+        them, by position or by name: every row decoded, then committed.  Up to 8
         rows have the bits of that many decode steps; longer prompts go
         through each step together (the same roundings, sums in another
         order)."""

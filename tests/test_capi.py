@@ -175,3 +175,37 @@ def test_packed_gemv_cache_evicts_least_recently_used(monkeypatch):
     assert (st["stores"], st["evictions"], st["resident_count"], st["resident_bytes"]) == (4, 2, 2, 800 << 10)
     native.reset_packed_gemv_cache()
     assert native.packed_gemv_cache_stats()["resident_count"] == 0
+
+
+def test_prefill_takes_its_weights_by_position_or_by_name(monkeypatch):
+    """dense_layer_prefill_packed_rows8 takes what the decode step takes, as
+    the loop over decode steps did: the weights as named arguments too."""
+    calls = []
+    session = object.__new__(native.NativeKvSession)
+    session.device, session.dtype, session.kv_width, session.max_seq_len = torch.device("cpu"), torch.float16, 8, 16
+    session._handle = None
+
+    class Lib:
+        kv_committed_length = kv_tentative_length = staticmethod(lambda handle, layer: 0)
+        kv_dense_layer_prefill_u16_ext_packed_rows8 = staticmethod(lambda *args: calls.append(args) or 0)
+
+    class Launch:
+        def __init__(self, lib, device):
+            pass
+
+        __enter__ = __exit__ = lambda self, *exc: None
+
+    session._lib = Lib
+    monkeypatch.setattr(native, "_launch", Launch)
+    H, inter = 16, 8
+    hidden = torch.zeros((3, H), dtype=torch.float16)
+    norms = [torch.ones(H, dtype=torch.float16) for _ in range(2)]
+    packed = [torch.zeros(n, dtype=torch.uint16) for n in (H * H, 8 * H, 8 * H, H * H, inter * H, inter * H, H * inter)]
+    kw = dict(hidden_size=H, intermediate_size=inter, num_heads=2, num_kv_heads=1, head_dim=8, rms_eps=1e-6,
+              rope_theta=1e4)
+    names = ["input_norm_weight", "post_norm_weight"] + [f"{n}_weight_packed" for n in "q k v o gate up down".split()]
+    session.dense_layer_prefill_packed_rows8(0, hidden, *norms, *packed, **kw)
+    session.dense_layer_prefill_packed_rows8(0, hidden, *norms, **dict(zip(names[2:], packed)), **kw)
+    session.dense_layer_prefill_packed_rows8(0, hidden, **dict(zip(names, norms + packed)), **kw)
+    out = len(calls[0]) - 7  # the output's address: a tensor of each call's own
+    assert len(calls) == 3 and all(a[:out] + a[out + 1:] == calls[0][:out] + calls[0][out + 1:] for a in calls)
