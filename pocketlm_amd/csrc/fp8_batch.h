@@ -8,7 +8,7 @@
 
 namespace plm {
 
-constexpr int kPanelOuts = 8;     // weights of one fp8_panel_linear call
+constexpr int kBatchOuts = 8;     // weights with outputs of their own in one call
 // Activation rows from which the panel kernel is the faster one, for a launch
 // over `rows` weight rows.  The skinny kernel's time grows with the rows (us,
 // bf16 / fp32 at 32, 64 and 128 rows: 7168x16384 53 / 80, 80 / 157, 155 / 310;
@@ -52,17 +52,18 @@ struct BatchRows {
     int waves = 0;                      // K blocks b = w, w + waves, ... are wave w's
     bool tiled = false;                 // weights in 8-row tiles
     BatchGroups groups;
-    // fp8_panel_linear: the weights w[0][i] of out_rows[i] rows each, to outs[i]
-    float* outs[kPanelOuts] = {};
-    int64_t out_rows[kPanelOuts] = {};
+    // outs[0] set: ngroups weights w[0][g] of out_rows[g] rows each (rows: the
+    // most), every activation row of each to outs[g][m][out_rows[g]]
+    float* outs[kBatchOuts] = {};
+    int64_t out_rows[kBatchOuts] = {};
 };
 
 int fp8_batch_rows(const BatchRows& p, hipStream_t st);
 
-// Prompt chunks (fp8_panel_kernel), the same bits: several linears over one
-// packed copy of the activations, and the SwiGLU MLP (gate_up's two weights,
-// then down's).
-int fp8_panel_linear(const BatchRows& p, int outs, hipStream_t st);
+// Prompt chunks (fp8_panel_kernel), the same bits: the linears of p.outs over
+// one packed copy of the activations, and the SwiGLU MLP (gate_up's two
+// weights, then down's).
+int fp8_panel_linear(const BatchRows& p, hipStream_t st);
 int fp8_panel_mlp(const BatchRows& gate_up, const BatchRows& down, hipStream_t st);
 
 // Waves of the down phase over nb K blocks (one group's): see fp8_down_kernel.

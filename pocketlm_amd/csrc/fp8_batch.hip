@@ -51,8 +51,10 @@ struct BatchArgs {
     int tiles;    // row tiles per group
     int nblocks;  // 128-column blocks per row
     int tiled;
+    int nouts;    // groups with rows and outputs of their own
+    int64_t out_rows[plm::kBatchOuts];
+    float* outs[plm::kBatchOuts];
 };
-
 
 // A workgroup owns 16 TA rows of each of its NWT weights; wave w of nw takes
 // the K blocks w, w + nw, ... for all 16 TB activation rows of a pass.
@@ -70,7 +72,15 @@ __global__ __launch_bounds__(64 * MAXW) void fp8_batch_kernel(const BatchArgs a)
     const int g = blockIdx.x / a.tiles;
     const int64_t row0 = static_cast<int64_t>(blockIdx.x - g * a.tiles) * 16 * TA;
     const int64_t count = a.count != nullptr ? a.count[g] : a.m;
-    const int64_t obase = a.base != nullptr ? a.base[g] : g * a.m;
+    int64_t obase = a.base != nullptr ? a.base[g] : g * a.m;
+    int64_t rows = a.rows;
+    float* out = a.out;
+    if (!SILU && a.nouts > 0) {
+        rows = a.out_rows[g];
+        out = a.outs[g];
+        obase = 0;
+        if (row0 >= rows) return;  // the whole workgroup
+    }
 
     const uint8_t* wrow[NT];
     const float* sp[NWT];
@@ -82,7 +92,7 @@ __global__ __launch_bounds__(64 * MAXW) void fp8_batch_kernel(const BatchArgs a)
 #pragma unroll
         for (int t = 0; t < TA; ++t) {
             // rows past the end read the last row; their results are dropped
-            const int64_t r = min(row0 + 16 * t + li, a.rows - 1);
+            const int64_t r = min(row0 + 16 * t + li, rows - 1);
             wrow[i * TA + t] =
                 a.w[i][g] + (a.tiled ? (r >> 3) * a.nblocks * 1024 + (r & 7) * 128 : r * a.K);
         }
@@ -221,7 +231,7 @@ __global__ __launch_bounds__(64 * MAXW) void fp8_batch_kernel(const BatchArgs a)
             const int r = e & 15, n = (e >> 4) & 15, tt = e >> 8;
             const int ta = tt % TA, tb = tt / TA;
             const int64_t row = row0 + 16 * ta + r, t = t0 + 16 * tb + n;
-            if (row >= a.rows || t >= count) continue;
+            if (row >= rows || t >= count) continue;
             float v[NWT];
 #pragma unroll
             for (int i = 0; i < NWT; ++i) {
@@ -230,11 +240,11 @@ __global__ __launch_bounds__(64 * MAXW) void fp8_batch_kernel(const BatchArgs a)
                 for (int w = 0; w < nw; ++w) s += rf[w * NT * TB * 256 + at];
                 v[i] = s;
             }
-            const int64_t o = (obase + t) * a.rows + row;
+            const int64_t o = (obase + t) * rows + row;
             if constexpr (SILU)
                 store_hplanes(a.hhi, a.hlo, o, plm_silu_mul(v[0], v[1]));
             else
-                a.out[o] = v[0];
+                out[o] = v[0];
         }
         __syncthreads();
     }
@@ -898,6 +908,14 @@ int plm::fp8_batch_rows(const BatchRows& p, hipStream_t st) {
     a.list = p.groups.list;
     a.nblocks = static_cast<int>(plm::ceil_div(p.K, 128));
     a.tiled = p.tiled ? 1 : 0;
+    if (p.outs[0] != nullptr) {
+        if (p.ngroups > kBatchOuts) return plm::fail(-2, "1..%d weights per call", kBatchOuts);
+        a.nouts = p.ngroups;
+        for (int g = 0; g < p.ngroups; ++g) {
+            a.outs[g] = p.outs[g];
+            a.out_rows[g] = p.out_rows[g];
+        }
+    }
     const bool grouped = p.groups.count != nullptr;
     const int64_t m = p.m;
     auto chunks = [&](int tb) { return grouped ? 1 : static_cast<int>(plm::ceil_div(m, 16 * tb)); };
@@ -919,17 +937,17 @@ int plm::fp8_batch_rows(const BatchRows& p, hipStream_t st) {
                         : launch<2, 2, 1, 1, false, kXF32, 8>(p, a, chunks(2), st);
 }
 
-int plm::fp8_panel_linear(const BatchRows& p, int outs, hipStream_t st) {
+int plm::fp8_panel_linear(const BatchRows& p, hipStream_t st) {
     const bool bf16 = p.xb != nullptr;
     const int tiles = panel_tiles(p.m, bf16);
     const int64_t first = panel_bytes(p.m, p.K, bf16);
     int64_t part = 0;
-    for (int i = 0; i < outs; ++i) part = std::max(part, panel_part(p.out_rows[i], false, tiles, p.waves, p.m));
+    for (int i = 0; i < p.ngroups; ++i) part = std::max(part, panel_part(p.out_rows[i], false, tiles, p.waves, p.m));
     char* x = static_cast<char*>(plm::workspace(static_cast<size_t>(first + part * 4)));
     if (x == nullptr) return -3;
     float* sums = reinterpret_cast<float*>(x + first);
     int code = pack_rows(p.x, p.xb, p.m, p.K, p.x_stride, x, st);
-    for (int i = 0; i < outs && code == 0; ++i) {
+    for (int i = 0; i < p.ngroups && code == 0; ++i) {
         PanelArgs a = panel_args(p, x, tiles);
         a.w[0] = p.w[0][i];
         a.s[0] = p.s[0][i];

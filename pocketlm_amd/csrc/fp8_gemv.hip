@@ -1750,61 +1750,48 @@ bool rows_fast_ok(const RowsProblem& p) {
 }
 
 // More than kMaxM activation rows on the vector path: whole MFMA tiles
-// (fp8_batch.hip), one launch per weight set; the same bits per row.
+// (fp8_batch.hip), the same bits per row.  One launch for the weights that
+// share the activations: linear, dual and many-linear; gate and up of up to
+// 64 experts.
 int run_rows_batch(const RowsProblem& p, hipStream_t st) {
-    const int outs = p.silu ? 1 : p.nwt;  // gate and up share a launch
-    const int n = p.nvar > 0 ? p.nvar : p.nwt;
-    int64_t widest = p.rows;
-    for (int i = 0; i < p.nvar; ++i) widest = std::max(widest, p.vrows[i]);
-    if (!p.silu && p.batch >= plm::panel_from(widest, p.xb != nullptr) && (p.nvar > 0 || p.ngroups == 1)) {
-        // linear, dual and many-linear: one packed copy of the activations
-        plm::BatchRows b;
-        for (int i = 0; i < n; ++i) {
+    plm::BatchRows b;
+    b.x = p.x;
+    b.xb = p.xb;
+    b.x_stride = p.x_stride;
+    b.K = p.K;
+    b.scale_cols = p.scale_cols;
+    b.m = p.batch;
+    b.tiled = p.tiled;
+    const int64_t nb = plm::ceil_div(p.K, 128);
+    b.waves = p.silu ? rows_waves<true>(nb) : rows_waves<false>(nb);
+    if (!p.silu) {
+        if (p.nvar == 0 && p.ngroups != 1) return plm::fail(-2, "bad dimensions");
+        b.ngroups = p.nvar > 0 ? p.nvar : p.nwt;
+        for (int i = 0; i < b.ngroups; ++i) {
             b.w[0][i] = p.nvar > 0 ? p.w[0][i] : p.w[i][0];
             b.s[0][i] = p.nvar > 0 ? p.s[0][i] : p.s[i][0];
             b.outs[i] = p.nvar > 0 ? p.vout[i] : p.out[i];
             b.out_rows[i] = p.nvar > 0 ? p.vrows[i] : p.rows;
+            b.rows = std::max(b.rows, b.out_rows[i]);
         }
-        b.x = p.x;
-        b.xb = p.xb;
-        b.x_stride = p.x_stride;
-        b.K = p.K;
-        b.scale_cols = p.scale_cols;
-        b.m = p.batch;
-        b.waves = rows_waves<false>(plm::ceil_div(p.K, 128));
-        b.tiled = p.tiled;
-        return plm::fp8_panel_linear(b, n, st);
+        if (p.batch >= plm::panel_from(b.rows, p.xb != nullptr)) return plm::fp8_panel_linear(b, st);
+        return plm::fp8_batch_rows(b, st);
     }
-    for (int i = 0; i < outs; ++i)
-        for (int g0 = 0; g0 < p.ngroups; g0 += p.nvar > 0 ? 1 : kMaxGroups) {
-            plm::BatchRows b;
-            b.ngroups = p.nvar > 0 ? 1 : std::min(kMaxGroups, p.ngroups - g0);
-            for (int g = 0; g < b.ngroups; ++g)
-                for (int k = 0; k < (p.silu ? 2 : 1); ++k) {
-                    b.w[k][g] = p.w[i + k][g0 + g];
-                    b.s[k][g] = p.s[i + k][g0 + g];
-                }
-            b.x = p.x;
-            b.xb = p.xb;
-            b.x_stride = p.x_stride;
-            b.rows = p.nvar > 0 ? p.vrows[g0] : p.rows;
-            b.K = p.K;
-            b.scale_cols = p.scale_cols;
-            b.m = p.batch;
-            const int64_t nb = plm::ceil_div(p.K, 128);
-            b.waves = p.silu ? rows_waves<true>(nb) : rows_waves<false>(nb);
-            b.tiled = p.tiled;
-            const int64_t goff = static_cast<int64_t>(g0) * p.batch * p.out_ld;
-            if (p.silu) {
-                uint16_t* planes = reinterpret_cast<uint16_t*>(p.out[0]);
-                b.hhi = planes + goff;
-                b.hlo = planes + static_cast<int64_t>(p.ngroups) * p.batch * p.out_ld + goff;
-            } else {
-                b.out = p.nvar > 0 ? p.vout[g0] : p.out[i] + goff;
+    b.rows = p.rows;
+    for (int g0 = 0; g0 < p.ngroups; g0 += kMaxGroups) {
+        b.ngroups = std::min(kMaxGroups, p.ngroups - g0);
+        for (int g = 0; g < b.ngroups; ++g)
+            for (int k = 0; k < 2; ++k) {
+                b.w[k][g] = p.w[k][g0 + g];
+                b.s[k][g] = p.s[k][g0 + g];
             }
-            const int code = plm::fp8_batch_rows(b, st);
-            if (code != 0) return code;
-        }
+        const int64_t goff = static_cast<int64_t>(g0) * p.batch * p.out_ld;
+        uint16_t* planes = reinterpret_cast<uint16_t*>(p.out[0]);
+        b.hhi = planes + goff;
+        b.hlo = planes + static_cast<int64_t>(p.ngroups) * p.batch * p.out_ld + goff;
+        const int code = plm::fp8_batch_rows(b, st);
+        if (code != 0) return code;
+    }
     return 0;
 }
 

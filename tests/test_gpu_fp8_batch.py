@@ -139,6 +139,47 @@ def test_other_entry_points_have_the_bits_of_one_row_calls(nat, dtype):
             assert torch.equal(rows[i:i + 1], one), i
 
 
+def _graph_us(calls):
+    """Microseconds a call on the device: the calls in a graph, fastest of five replays."""
+    graph = torch.cuda.CUDAGraph()
+    for call in calls:
+        call()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        kept = [call() for call in calls]
+    times = []
+    for _ in range(6):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        graph.replay()
+        end.record()
+        torch.cuda.synchronize()
+        times.append(start.elapsed_time(end) * 1e3 / len(kept))
+    return min(times[1:])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("cols,outs", [(7168, (2048, 2048)), (1024, (512, 512)), (7168, (1536, 576)),
+                                       (2048, (1024, 576, 1024))])
+def test_twelve_rows_take_no_longer_than_eight_and_four(nat, cols, outs, dtype):
+    """One call is the faster one (0.4 to 0.8 of the time of two; the bar is
+    that it is not the slower one)."""
+    sets = [[_fp8(n, cols, 10 * i + j) for j, n in enumerate(outs)] for i in range(8)]
+    x = _x(12, cols, 1, dtype)
+
+    def call(weights, rows):
+        if len(outs) == 1:
+            return nat.fp8_e4m3_block_linear_f32(*weights[0], rows)
+        if outs[0] == outs[-1] and len(outs) == 2:
+            return nat.fp8_e4m3_block_dual_linear_f32(*weights[0], *weights[1], rows)
+        return nat.fp8_e4m3_block_linear_many_f32(weights, rows)
+
+    one = _graph_us([lambda w=w: call(w, x) for w in sets])
+    two = _graph_us([lambda w=w: (call(w, x[:8]), call(w, x[8:])) for w in sets])
+    print(cols, outs, dtype, one, two, flush=True)
+    assert one <= two
+
+
 def test_prompt_calls_captured_cold(nat):
     """The first panel-kernel calls on a stream, made under capture (scratch
     and the large-LDS setting included): every replay, with eager work in
