@@ -64,6 +64,13 @@ __global__ __launch_bounds__(64 * MAXW) void fp8_batch_kernel(const BatchArgs a)
     constexpr int PL = XM == kXPlanes ? 2 : 1;  // planes of the activations, with accumulators of their own
     constexpr bool XB = XM != kXF32;
     constexpr int XE = XB ? 2 : 4;
+    // Whether a ragged block's columns past K are masked before its first
+    // matrix instruction, and not half by half: with the branch between one and
+    // the read of its result ROCm 7.2's compiler left out the wait states in a
+    // 16-row instance (wrong sums after a NaN byte); in the wider ones it does
+    // not, and there the early mask is slower (the 4096/2048 MLP at 17 rows 24
+    // -> 32 us).
+    constexpr bool EARLY = TA == 1 && !SILU;
     extern __shared__ plm_f32x4 red[];  // [wave][tile][lane]
     const int nw = blockDim.x >> 6;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -157,6 +164,20 @@ __global__ __launch_bounds__(64 * MAXW) void fp8_batch_kernel(const BatchArgs a)
                     float sc[NWT];
 #pragma unroll
                     for (int n = 0; n < NWT; ++n) sc[n] = lane_value(sv[n], k);
+                    // columns past K add nothing
+                    auto clip = [](plm_u32x4& v, bool in) { v = in ? v : plm_u32x4{0, 0, 0, 0}; };
+                    if (EARLY && ragged) {
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            const bool in = b * 128 + 64 * h + 16 * qd < K;
+#pragma unroll
+                            for (int t = 0; t < NT; ++t) clip(q[slot][h][t], in);
+#pragma unroll
+                            for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+                                for (int i = 0; i < (XB ? 2 : 4); ++i) clip(x[slot][h][0][tb].v[i], in);
+                        }
+                    }
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {
                         const bool in = !ragged || b * 128 + 64 * h + 16 * qd < K;
@@ -164,7 +185,7 @@ __global__ __launch_bounds__(64 * MAXW) void fp8_batch_kernel(const BatchArgs a)
 #pragma unroll
                         for (int t = 0; t < NT; ++t) {
                             plm_u32x4 qv = q[slot][h][t];
-                            if (ragged) qv = in ? qv : plm_u32x4{0, 0, 0, 0};
+                            if (!EARLY && ragged) clip(qv, in);
                             weights_to_bf16(SAN ? zero_nan_bytes(qv) : qv, a0[t], a1[t]);
                         }
 #pragma unroll
@@ -172,10 +193,9 @@ __global__ __launch_bounds__(64 * MAXW) void fp8_batch_kernel(const BatchArgs a)
 #pragma unroll
                             for (int pl = 0; pl < PL; ++pl) {
                                 XPiece<XB> xv = x[slot][h][pl][tb];
-                                if (ragged) {
+                                if (!EARLY && ragged) {
 #pragma unroll
-                                    for (int i = 0; i < (XB ? 2 : 4); ++i)
-                                        xv.v[i] = in ? xv.v[i] : plm_u32x4{0, 0, 0, 0};
+                                    for (int i = 0; i < (XB ? 2 : 4); ++i) clip(xv.v[i], in);
                                 }
                                 const BOperands<XB, SAN> bo(xv);
 #pragma unroll
@@ -927,14 +947,29 @@ int plm::fp8_batch_rows(const BatchRows& p, hipStream_t st) {
                             : launch<1, 2, 1, 2, true, kXF32, 4>(p, a, chunks(2), st);
     }
     if (xm == kXPlanes) return launch<2, 1, 1, 1, false, kXPlanes, 16>(p, a, chunks(1), st);
-    if (m <= 16)
-        return xm == kXBf16 ? launch<2, 1, 2, 1, false, kXBf16, 8>(p, a, chunks(1), st)
-                            : launch<2, 1, 2, 1, false, kXF32, 8>(p, a, chunks(1), st);
-    if (m <= 32)
-        return xm == kXBf16 ? launch<2, 2, 2, 1, false, kXBf16, 8>(p, a, chunks(2), st)
-                            : launch<2, 2, 1, 1, false, kXF32, 8>(p, a, chunks(2), st);
-    return xm == kXBf16 ? launch<2, 4, 1, 1, false, kXBf16, 8>(p, a, chunks(4), st)
-                        : launch<2, 2, 1, 1, false, kXF32, 8>(p, a, chunks(2), st);
+    // 16 weight rows a workgroup while that still leaves at most one for each
+    // compute unit, else 32: a workgroup's time is its chain of K blocks, and
+    // half of the rows take less than half of the work (2048x7168 at 9 and 16
+    // bf16 rows, us: 15.7 and 18.2 -> 11.4 and 13.6, at 64 37.9 -> 32.8; fp32
+    // 19.8 and 25.1 -> 15.4 and 20.7).  Past one round the wider tile wins:
+    // 7168x2048 at 16 rows 8.3 against 9.5, 4096x7168 at 65 39 against 48.
+    const int tb = m <= 16 ? 1 : (m <= 32 || xm == kXF32 ? 2 : 4);
+    int64_t narrow = 0;
+    for (int g = 0; g < p.ngroups; ++g) narrow += plm::ceil_div(p.outs[0] != nullptr ? p.out_rows[g] : p.rows, 16);
+    if (narrow * chunks(tb) <= plm::cu_count()) {
+        if (xm == kXBf16)
+            return tb == 1 ? launch<1, 1, 2, 1, false, kXBf16, 8>(p, a, chunks(1), st)
+                           : (tb == 2 ? launch<1, 2, 2, 1, false, kXBf16, 8>(p, a, chunks(2), st)
+                                      : launch<1, 4, 2, 1, false, kXBf16, 8>(p, a, chunks(4), st));
+        return tb == 1 ? launch<1, 1, 2, 1, false, kXF32, 8>(p, a, chunks(1), st)
+                       : launch<1, 2, 2, 1, false, kXF32, 8>(p, a, chunks(2), st);
+    }
+    if (xm == kXBf16)
+        return tb == 1 ? launch<2, 1, 2, 1, false, kXBf16, 8>(p, a, chunks(1), st)
+                       : (tb == 2 ? launch<2, 2, 2, 1, false, kXBf16, 8>(p, a, chunks(2), st)
+                                  : launch<2, 4, 1, 1, false, kXBf16, 8>(p, a, chunks(4), st));
+    return tb == 1 ? launch<2, 1, 2, 1, false, kXF32, 8>(p, a, chunks(1), st)
+                   : launch<2, 2, 1, 1, false, kXF32, 8>(p, a, chunks(2), st);
 }
 
 int plm::fp8_panel_linear(const BatchRows& p, hipStream_t st) {

@@ -45,7 +45,7 @@ def _rows_of(fn, x, at):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("rows,cols", [(72, 144), (200, 2064), (576, 7168), (130, 1024)])
+@pytest.mark.parametrize("rows,cols", [(72, 144), (200, 2064), (576, 7168), (130, 1024), (4200, 144)])
 def test_rows_have_the_bits_of_one_row_calls(nat, rows, cols, dtype):
     w, s = _fp8(rows, cols, rows + cols, nan_at=[(rows - 1, 17)])
     w2, s2 = _fp8(rows, cols, rows + cols + 1)
@@ -160,7 +160,7 @@ def _graph_us(calls):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("cols,outs", [(7168, (2048, 2048)), (1024, (512, 512)), (7168, (1536, 576)),
-                                       (2048, (1024, 576, 1024))])
+                                       (2048, (1024, 576, 1024)), (7168, (576,)), (7168, (2048,)), (1024, (2048,))])
 def test_twelve_rows_take_no_longer_than_eight_and_four(nat, cols, outs, dtype):
     """One call is the faster one (0.4 to 0.8 of the time of two; the bar is
     that it is not the slower one)."""
