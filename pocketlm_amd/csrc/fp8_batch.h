@@ -5,19 +5,11 @@
 #include <cstdint>
 
 #include "common.h"
+#include "fp8_plan.h"
 
 namespace plm {
 
 constexpr int kBatchOuts = 8;     // weights with outputs of their own in one call
-// Activation rows from which the panel kernel is the faster one, for a launch
-// over `rows` weight rows.  The skinny kernel's time grows with the rows (us,
-// bf16 / fp32 at 32, 64 and 128 rows: 7168x16384 53 / 80, 80 / 157, 155 / 310;
-// 2048x7168 25 / 39, 38 / 39, 39 / 39), the panel kernel's hardly does
-// (105 / 88, 23 / 23): they cross at about 80 / 36 rows of a tall weight and
-// 32 / 14 of a short one, 68 / 36 for 24576x1536.
-constexpr int64_t panel_from(int64_t rows, bool bf16) {
-    return bf16 ? (rows >= 4096 ? 65 : 33) : (rows >= 4096 ? 33 : 17);
-}
 constexpr int kBatchGroups = 64;  // weights per launch (their addresses travel as kernel arguments)
 
 // Where the tokens of a grouped launch are, on the device (all indexed by

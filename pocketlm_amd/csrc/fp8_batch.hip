@@ -445,7 +445,8 @@ __global__ __launch_bounds__(kPairThreads) void pair_sum_kernel(const float* __r
 // or from the gate/up launch's epilogue.  Rows past m hold anything (their
 // columns are dropped); columns past K are zero.
 
-constexpr int kPanelCols = 8;      // column tiles per workgroup
+using plm::kPanelCols;
+using plm::panel_tiles;
 constexpr int kTileBytes = 4096;   // one column tile of one block
 
 struct PanelArgs {
@@ -783,12 +784,6 @@ __global__ __launch_bounds__(256) void fp8_pack_rows_kernel(const char* __restri
     }
 }
 
-// Column tiles of m activation rows (two per token tile for hi and lo), in
-// whole workgroups.
-int panel_tiles(int64_t m, bool one_plane) {
-    return static_cast<int>(plm::ceil_div(plm::ceil_div(m, 16) * (one_plane ? 1 : 2), kPanelCols)) * kPanelCols;
-}
-
 int64_t panel_bytes(int64_t m, int64_t K, bool one_plane) {
     return plm::ceil_div(K, 128) * panel_tiles(m, one_plane) * kTileBytes;
 }
@@ -833,38 +828,21 @@ int launch_panel(const PanelArgs& args, hipStream_t st) {
     return plm::check_launch("fp8 panel sum");
 }
 
-// Workgroups of 128 weight rows where that leaves one for every compute unit,
-// else of 64, and where those leave many units idle the K slots split over
-// two workgroups a unit: a workgroup alone takes 1.2 us a block whatever the
-// launch, so 7168x16384 at 128 rows goes from 161 us (112 workgroups) to 105,
-// 2048x7168 from 77 to 25; 224 workgroups are better left whole (7168x16384
-// at 256 rows 167 us, split in three 214).
-constexpr int64_t kPanelWhole = 192;   // workgroups from which the slots stay together
-constexpr int64_t kPanelGroups = 512;
-
-int64_t panel_groups(int64_t rows, bool silu, int x_tiles, int wr) {
-    return plm::ceil_div(rows, (silu ? 32 : 64) * wr) * (x_tiles / kPanelCols);
-}
-
-int panel_splits(int64_t rows, bool silu, int x_tiles, int waves) {
-    const int64_t groups = panel_groups(rows, silu, x_tiles, 1);
-    if (groups >= kPanelWhole) return 1;
-    return static_cast<int>(std::min<int64_t>(waves, plm::ceil_div(kPanelGroups, groups)));
-}
-
 // Floats of the slots' sums.
 int64_t panel_part(int64_t rows, bool silu, int x_tiles, int waves, int64_t m) {
-    return panel_splits(rows, silu, x_tiles, waves) == 1 ? 0 : waves * m * rows * (silu ? 2 : 1);
+    const int splits = plm::panel_plan(rows, silu, x_tiles, waves, plm::cu_count()).splits;
+    return splits == 1 ? 0 : waves * m * rows * (silu ? 2 : 1);
 }
 
 template <bool SILU, int MODE>
 int launch_panel_rows(const PanelArgs& args, float* part, hipStream_t st) {
     PanelArgs a = args;
-    a.splits = panel_splits(a.rows, SILU, a.x_tiles, a.waves);
+    const plm::PanelPlan plan = plm::panel_plan(a.rows, SILU, a.x_tiles, a.waves, plm::cu_count());
+    a.splits = plan.splits;
     a.part = part;
     a.part_ld = a.rows * (SILU ? 2 : 1);
-    if (panel_groups(a.rows, SILU, a.x_tiles, 2) >= plm::cu_count()) return launch_panel<2, SILU, MODE>(a, st);
-    return a.splits == 1 ? launch_panel<1, SILU, MODE>(a, st) : launch_panel<1, SILU, MODE, true>(a, st);
+    if (plan.wr == 2) return launch_panel<2, SILU, MODE>(a, st);
+    return plan.splits == 1 ? launch_panel<1, SILU, MODE>(a, st) : launch_panel<1, SILU, MODE, true>(a, st);
 }
 
 PanelArgs panel_args(const plm::BatchRows& p, const char* x, int x_tiles) {
