@@ -1774,7 +1774,7 @@ int run_rows_batch(const RowsProblem& p, hipStream_t st) {
             b.out_rows[i] = p.nvar > 0 ? p.vrows[i] : p.rows;
             b.rows = std::max(b.rows, b.out_rows[i]);
         }
-        if (p.batch >= plm::panel_from(b.rows, p.xb != nullptr)) return plm::fp8_panel_linear(b, st);
+        if (p.batch >= plm::panel_from(b.rows, nb, b.ngroups, p.xb != nullptr)) return plm::fp8_panel_linear(b, st);
         return plm::fp8_batch_rows(b, st);
     }
     b.rows = p.rows;
@@ -2161,8 +2161,9 @@ int mlp_impl(const uint8_t* gate_weight, const float* gate_scale_inv, const uint
     const uint64_t dp = reinterpret_cast<uintptr_t>(down_weight), dsp = reinterpret_cast<uintptr_t>(down_scale_inv);
     hipStream_t st = plm::current_stream();
     const void* x = hidden.f32 != nullptr ? static_cast<const void*>(hidden.f32) : hidden.bf16;
-    if (batch >= plm::panel_from(2 * intermediate_rows, hidden.bf16 != nullptr) && intermediate_rows % 16 == 0 && hidden_cols % 16 == 0 && plm::aligned16(x) &&
-        plm::aligned16(gate_weight) && plm::aligned16(up_weight) && plm::aligned16(down_weight)) {
+    const bool aligned = intermediate_rows % 16 == 0 && hidden_cols % 16 == 0 && plm::aligned16(x) &&
+                         plm::aligned16(gate_weight) && plm::aligned16(up_weight) && plm::aligned16(down_weight);
+    if (aligned && batch >= plm::panel_mlp_from(hidden_cols, intermediate_rows, hidden.bf16 != nullptr)) {
         plm::BatchRows gu, dn;
         gu.w[0][0] = gate_weight;
         gu.w[1][0] = up_weight;

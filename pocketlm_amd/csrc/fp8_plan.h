@@ -8,14 +8,47 @@ namespace plm {
 
 constexpr int kPanelCols = 8;  // column tiles of 16 per workgroup of the panel kernel
 
-// Activation rows from which the panel kernel is the faster one, for a launch
-// over `rows` weight rows.  The skinny kernel's time grows with the rows (us,
-// bf16 / fp32 at 32, 64 and 128 rows: 7168x16384 53 / 80, 80 / 157, 155 / 310;
-// 2048x7168 25 / 39, 38 / 39, 39 / 39), the panel kernel's hardly does
-// (105 / 88, 23 / 23): they cross at about 80 / 36 rows of a tall weight and
-// 32 / 14 of a short one, 68 / 36 for 24576x1536.
-constexpr int64_t panel_from(int64_t rows, bool bf16) {
-    return bf16 ? (rows >= 4096 ? 65 : 33) : (rows >= 4096 ? 33 : 17);
+// Activation rows from which the panel kernel is the faster one, for a launch of
+// `outs` weights, the largest of `rows` rows, `blocks` blocks of 128 columns
+// each.  The skinny kernel takes one launch, its time a step for each 16, 32 or
+// 64 rows and for each round of workgroups; the panel kernel takes two to three
+// launches (10 us and more) per weight but hardly grows.  Skinny / panel, us:
+//   bf16   2048x7168 at 32, 33, 64 rows 20/21, 23/21, 33/23   2048x2048 at 64, 256 13/15, 16/24
+//          7168x16384 at 64, 65 83/97, 121/97   4096x4096 at 64, 128, 192 21/26, 26/28, 48/43
+//          24576x1536 at 64, 65 42/46, 62/46    7168x2048 at 64, 128, 192 17/30, 31/36, 45/31
+//          2048 + 2048 x7168 at 64, 128, 192 34/41, 40/43, 77/67
+//   fp32   2048x7168 at 16, 17 21/20, 24/20     2048x2048 at 64, 192, 256 12/14, 28/26, 28/27
+//          7168x16384 at 32, 33 85/90, 122/90   4096x4096 at 32, 33, 65 21/24, 26/24, 38/35
+//          24576x1536 at 32, 33 38/41, 56/42    7168x2048 at 64, 65 29/29, 36/27
+//          2048 + 2048 x7168 at 64, 65, 96 40/39, 56/59, 76/60
+//   2048 + 576 + 2048 x7168: bf16 at 64, 96, 128 40/58, 59/59, 76/60, fp32 at 33, 48, 64 41/53, 60/54, 74/55
+//   4096 + 1024 + 1024 x4096: bf16 at 128, 192 50/57, 72/73, fp32 at 64, 96 47/48, 72/62
+constexpr int64_t panel_from(int64_t rows, int64_t blocks, int outs, bool bf16) {
+    if (outs > 1) {
+        if (blocks < 32) return !bf16 && rows >= 2048 ? 193 : 257;
+        return blocks >= 56 ? (bf16 ? 97 : 41) : (bf16 ? 193 : 65);
+    }
+    if (blocks < 32) {
+        if (rows >= 16384) return bf16 ? 65 : 33;
+        if (rows >= 4096 && blocks >= 16) return bf16 ? 129 : 65;
+        return !bf16 && (rows >= 4096 || blocks >= 16) ? 193 : 257;
+    }
+    if (rows < 4096) return bf16 ? 33 : 17;
+    return bf16 ? (blocks >= 56 ? 65 : 129) : 33;
+}
+
+// The same for the SwiGLU MLP.  Skinny / panel, us: bf16 7168/2048 at 64, 65
+// 61/61, 78/61, 4096/1024 at 128, 129 35/39, 45/39, 1024/2048 at 256, 257 47/47,
+// 56/42, 1024/512 at 512 25/32; fp32 7168/2048 at 32, 33 57/57, 64/58, 4096/1024
+// at 64, 96 34/34, 39/37, 2048/1024 at 192, 256 39/41, 42/41, 7168/512 at 24, 32
+// 39/37, 44/38: the skinny kernels' time grows with rows x weight (below 1024
+// intermediate rows with rows x hidden), the panel's extra launches cost 10 to
+// 15 us.
+constexpr int64_t panel_mlp_from(int64_t hidden, int64_t inter, bool bf16) {
+    if (!bf16 && hidden >= 7168 && inter < 1024) return 17;
+    const int64_t size = hidden * (inter > 1024 ? inter : 1024);
+    const int64_t rows = (int64_t(1) << (bf16 ? 29 : 28)) / size + 1, least = bf16 ? 65 : 33;
+    return rows > least ? rows : least;
 }
 
 // Column tiles of m activation rows (two per token tile for hi and lo), in

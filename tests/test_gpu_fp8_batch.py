@@ -10,6 +10,9 @@ each), rel-L2 2e-5.
 
 from __future__ import annotations
 
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -119,8 +122,8 @@ def test_other_entry_points_have_the_bits_of_one_row_calls(nat, dtype):
     weights = [_fp8(rows, 400, rows) for rows in (24, 136, 300)]
     packed = [nat.pack_fp8_tiles8(w) for w, _s in weights]
     items = [(*_fp8(48, 144, 3 * e), *_fp8(48, 144, 3 * e + 1), *_fp8(144, 48, 3 * e + 2)) for e in range(66)]
-    route = torch.rand((66, 150), generator=torch.Generator().manual_seed(1)).cuda()
-    for m in (9, 20, 40, 150):
+    route = torch.rand((66, 260), generator=torch.Generator().manual_seed(1)).cuda()
+    for m in (9, 20, 40, 150, 260):
         print("entry points", m, dtype, flush=True)
         x = _x(m, 400, m, dtype)
         for (w, s), p, y in zip(weights, packed, nat.fp8_e4m3_block_linear_many_f32(weights, x)):
@@ -180,17 +183,54 @@ def test_twelve_rows_take_no_longer_than_eight_and_four(nat, cols, outs, dtype):
     assert one <= two
 
 
-def test_prompt_calls_captured_cold(nat):
-    """The first panel-kernel calls on a stream, made under capture (scratch
+# Shapes of the prompt-chunk kernel, LONG rows each: (rows, cols) of a linear,
+# (inter, hid) of an MLP.  On 256 compute units they reach every instance of
+# it: 64- and 128-row workgroups, K slots together and split, for linear, gate +
+# up and down, in both types (tests/test_fp8_plan.py holds them to that); no
+# size is a multiple of a tile.
+LONG = 509
+LONG_LINEARS = [(200, 2064), (8100, 144), (4000, 144), (3100, 272), (1500, 272), (328, 7184)]
+LONG_MLPS = [(4048, 272), (1552, 720), (784, 1040), (144, 2064), (144, 4000), (272, 1520)]
+LONG_ROWS = (0, 15, 16, 127, 128, 300, 496, 507, 508)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,cols", LONG_LINEARS)
+def test_long_prompt_chunks_have_the_bits_of_one_row_calls(nat, rows, cols, dtype):
+    w, s = _fp8(rows, cols, rows, nan_at=[(rows - 1, 17), (0, cols - 1)])
+    x = _x(LONG, cols, cols, dtype)
+    y = nat.fp8_e4m3_block_linear_f32(w, s, x)
+    assert torch.isfinite(y).all()
+    assert torch.equal(y[list(LONG_ROWS)], _rows_of(lambda r: nat.fp8_e4m3_block_linear_f32(w, s, r), x, LONG_ROWS))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("inter,hid", LONG_MLPS)
+def test_long_prompt_chunks_of_the_mlp_have_the_bits_of_one_row_calls(nat, inter, hid, dtype):
+    args = [*_fp8(inter, hid, 1, nan_at=[(inter - 1, 5)]), *_fp8(inter, hid, 2, nan_at=[(3, hid - 1)]),
+            *_fp8(hid, inter, 3, nan_at=[(hid - 1, 0)])]
+    x = _x(LONG, hid, hid, dtype)
+    y = nat.fp8_e4m3_block_mlp_f32(*args, x)
+    assert torch.isfinite(y).all()
+    assert torch.equal(y[list(LONG_ROWS)], _rows_of(lambda r: nat.fp8_e4m3_block_mlp_f32(*args, r), x, LONG_ROWS))
+
+
+def test_prompt_calls_captured_cold():
+    """The first panel-kernel calls of a process, made under capture (scratch
     and the large-LDS setting included): every replay, with eager work in
     between, equals the eager call."""
+    subprocess.run([sys.executable, __file__], check=True, timeout=110)
+
+
+def _captured_cold(nat):
     w, s = _fp8(328, 1040, 5)
     mlp = [*_fp8(272, 1040, 6), *_fp8(272, 1040, 7), *_fp8(1040, 272, 8)]
     items = [(*_fp8(144, 1040, 3 * e), *_fp8(144, 1040, 3 * e + 1), *_fp8(1040, 144, 3 * e + 2)) for e in range(5)]
-    x = _x(70, 1040, 9, torch.float32)
-    pi = torch.arange(140, device="cuda") % 5
-    pr = torch.arange(140, device="cuda") // 2
-    pw = torch.rand(140, generator=torch.Generator().manual_seed(2)).cuda()
+    rows = 300
+    x = _x(rows, 1040, 9, torch.float32)
+    pi = torch.arange(2 * rows, device="cuda") % 5
+    pr = torch.arange(2 * rows, device="cuda") // 2
+    pw = torch.rand(2 * rows, generator=torch.Generator().manual_seed(2)).cuda()
 
     def step():
         return (nat.fp8_e4m3_block_linear_f32(w, s, x), nat.fp8_e4m3_block_mlp_f32(*mlp, x),
@@ -201,9 +241,15 @@ def test_prompt_calls_captured_cold(nat):
     with torch.cuda.graph(graph):
         captured = step()
     for trial in range(3):
-        x.copy_(_x(70, 1040, 20 + trial, torch.float32))
+        x.copy_(_x(rows, 1040, 20 + trial, torch.float32))
         graph.replay()
         torch.cuda.synchronize()
         got = [t.clone() for t in captured]
         for a, b in zip(got, step()):
             assert torch.equal(a, b), trial
+
+
+if __name__ == "__main__":
+    from pocketlm_amd import native
+
+    _captured_cold(native)
