@@ -845,7 +845,7 @@ int launch_panel_rows(const PanelArgs& args, float* part, hipStream_t st) {
     return plan.splits == 1 ? launch_panel<1, SILU, MODE>(a, st) : launch_panel<1, SILU, MODE, true>(a, st);
 }
 
-PanelArgs panel_args(const plm::BatchRows& p, const char* x, int x_tiles) {
+PanelArgs panel_args(const plm::BatchRows& p, const char* x, int x_tiles, int64_t m) {
     PanelArgs a;
     std::memset(&a, 0, sizeof(a));
     for (int i = 0; i < (p.hhi != nullptr ? 2 : 1); ++i) {
@@ -857,7 +857,7 @@ PanelArgs panel_args(const plm::BatchRows& p, const char* x, int x_tiles) {
     a.rows = p.rows;
     a.K = p.K;
     a.scale_cols = p.scale_cols;
-    a.m = p.m;
+    a.m = m;
     a.nblocks = static_cast<int>(plm::ceil_div(p.K, 128));
     a.waves = p.waves;
     a.x_tiles = x_tiles;
@@ -950,30 +950,44 @@ int plm::fp8_batch_rows(const BatchRows& p, hipStream_t st) {
                    : launch<2, 2, 1, 1, false, kXF32, 8>(p, a, chunks(2), st);
 }
 
-int plm::fp8_panel_linear(const BatchRows& p, hipStream_t st) {
+namespace {
+
+// Activation rows of a call beyond kPanelPass go in passes over the weights, so
+// that its packed copy stays a bounded part of the thread's scratch (268 MB for
+// 16384 fp32 columns): one read of a weight in 4096 rows is nothing.
+constexpr int64_t kPanelPass = 4096;
+
+template <class Pass>
+int in_passes(int64_t m, Pass pass) {
+    int code = 0;
+    for (int64_t m0 = 0; m0 < m && code == 0; m0 += kPanelPass) code = pass(m0, std::min(kPanelPass, m - m0));
+    return code;
+}
+
+int panel_linear_rows(const plm::BatchRows& p, int64_t m0, int64_t m, hipStream_t st) {
     const bool bf16 = p.xb != nullptr;
-    const int tiles = panel_tiles(p.m, bf16);
-    const int64_t first = panel_bytes(p.m, p.K, bf16);
+    const int tiles = panel_tiles(m, bf16);
+    const int64_t first = panel_bytes(m, p.K, bf16);
     int64_t part = 0;
-    for (int i = 0; i < p.ngroups; ++i) part = std::max(part, panel_part(p.out_rows[i], false, tiles, p.waves, p.m));
+    for (int i = 0; i < p.ngroups; ++i) part = std::max(part, panel_part(p.out_rows[i], false, tiles, p.waves, m));
     char* x = static_cast<char*>(plm::workspace(static_cast<size_t>(first + part * 4)));
     if (x == nullptr) return -3;
     float* sums = reinterpret_cast<float*>(x + first);
-    int code = pack_rows(p.x, p.xb, p.m, p.K, p.x_stride, x, st);
+    const int64_t skip = m0 * p.x_stride;
+    int code = pack_rows(bf16 ? nullptr : p.x + skip, bf16 ? p.xb + skip : nullptr, m, p.K, p.x_stride, x, st);
     for (int i = 0; i < p.ngroups && code == 0; ++i) {
-        PanelArgs a = panel_args(p, x, tiles);
+        PanelArgs a = panel_args(p, x, tiles, m);
         a.w[0] = p.w[0][i];
         a.s[0] = p.s[0][i];
-        a.out = p.outs[i];
+        a.out = p.outs[i] + m0 * p.out_rows[i];
         a.rows = p.out_rows[i];
         code = bf16 ? launch_panel_rows<false, kXBf16>(a, sums, st) : launch_panel_rows<false, kXF32>(a, sums, st);
     }
     return code;
 }
 
-int plm::fp8_panel_mlp(const BatchRows& gate_up, const BatchRows& down, hipStream_t st) {
+int panel_mlp_rows(const plm::BatchRows& gate_up, const plm::BatchRows& down, int64_t m0, int64_t m, hipStream_t st) {
     const bool bf16 = gate_up.xb != nullptr;
-    const int64_t m = gate_up.m;
     const int tiles = panel_tiles(m, bf16), out_tiles = panel_tiles(m, false);
     const int64_t first = panel_bytes(m, gate_up.K, bf16), second = panel_bytes(m, down.K, false);
     const int64_t part = std::max(panel_part(gate_up.rows, true, tiles, gate_up.waves, m),
@@ -981,9 +995,11 @@ int plm::fp8_panel_mlp(const BatchRows& gate_up, const BatchRows& down, hipStrea
     char* x = static_cast<char*>(plm::workspace(static_cast<size_t>(first + second + part * 4)));
     if (x == nullptr) return -3;
     float* sums = reinterpret_cast<float*>(x + first + second);
-    int code = pack_rows(gate_up.x, gate_up.xb, m, gate_up.K, gate_up.x_stride, x, st);
+    const int64_t skip = m0 * gate_up.x_stride;
+    int code = pack_rows(bf16 ? nullptr : gate_up.x + skip, bf16 ? gate_up.xb + skip : nullptr, m, gate_up.K,
+                         gate_up.x_stride, x, st);
     if (code != 0) return code;
-    PanelArgs a = panel_args(gate_up, x, tiles);
+    PanelArgs a = panel_args(gate_up, x, tiles, m);
     for (int i = 0; i < 2; ++i) {
         a.w[i] = gate_up.w[i][0];
         a.s[i] = gate_up.s[i][0];
@@ -992,7 +1008,19 @@ int plm::fp8_panel_mlp(const BatchRows& gate_up, const BatchRows& down, hipStrea
     a.out_tiles = out_tiles;
     code = bf16 ? launch_panel_rows<true, kXBf16>(a, sums, st) : launch_panel_rows<true, kXF32>(a, sums, st);
     if (code != 0) return code;
-    return launch_panel_rows<false, kXPlanes>(panel_args(down, x + first, out_tiles), sums, st);
+    PanelArgs d = panel_args(down, x + first, out_tiles, m);
+    d.out += m0 * down.rows;
+    return launch_panel_rows<false, kXPlanes>(d, sums, st);
+}
+
+}  // namespace
+
+int plm::fp8_panel_linear(const BatchRows& p, hipStream_t st) {
+    return in_passes(p.m, [&](int64_t m0, int64_t m) { return panel_linear_rows(p, m0, m, st); });
+}
+
+int plm::fp8_panel_mlp(const BatchRows& gate_up, const BatchRows& down, hipStream_t st) {
+    return in_passes(gate_up.m, [&](int64_t m0, int64_t m) { return panel_mlp_rows(gate_up, down, m0, m, st); });
 }
 
 int plm::fp8_batch_pairs(const PairProblem& p, hipStream_t st) {

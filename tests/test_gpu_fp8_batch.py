@@ -12,12 +12,14 @@ from __future__ import annotations
 
 import subprocess
 import sys
+import threading
 
 import numpy as np
 import pytest
 import torch
 
 from conftest import rel_l2
+from pocketlm_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -213,6 +215,34 @@ def test_long_prompt_chunks_of_the_mlp_have_the_bits_of_one_row_calls(nat, inter
     y = nat.fp8_e4m3_block_mlp_f32(*args, x)
     assert torch.isfinite(y).all()
     assert torch.equal(y[list(LONG_ROWS)], _rows_of(lambda r: nat.fp8_e4m3_block_mlp_f32(*args, r), x, LONG_ROWS))
+
+
+def test_scratch_of_a_very_long_chunk_is_bounded(nat):
+    """A linear and an MLP of 20000 rows (five passes of 4096): scratch as for
+    4096 rows (its packed fp32 copy is 4096 x 384 x 4 = 6.3 MB, the MLP's with
+    its intermediate 25 MB, in arenas of whole MB that are kept when a larger
+    one replaces them), every row with the bits of one-row calls."""
+    w, s = _fp8(200, 272, 1)
+    mlp = [*_fp8(272, 1040, 2), *_fp8(272, 1040, 3), *_fp8(1040, 272, 4)]
+    x, h = _x(20000, 272, 5, torch.float32), _x(20000, 1040, 6, torch.float32)
+    at = (0, 4095, 4096, 8191, 8192, 19999)
+    box = {}
+
+    def run():
+        lib = _lib.load()
+        box["linear"] = nat.fp8_e4m3_block_linear_f32(w, s, x)
+        box["linear bytes"] = lib.pocketlm_scratch_bytes()
+        box["mlp"] = nat.fp8_e4m3_block_mlp_f32(*mlp, h)
+        box["mlp bytes"] = lib.pocketlm_scratch_bytes()
+        torch.cuda.synchronize()
+        lib.pocketlm_release_scratch()
+
+    thread = threading.Thread(target=run)
+    thread.start()
+    thread.join()
+    assert box["linear bytes"] <= 8 << 20 and box["mlp bytes"] <= 48 << 20, box
+    assert torch.equal(box["linear"][list(at)], _rows_of(lambda r: nat.fp8_e4m3_block_linear_f32(w, s, r), x, at))
+    assert torch.equal(box["mlp"][list(at)], _rows_of(lambda r: nat.fp8_e4m3_block_mlp_f32(*mlp, r), h, at))
 
 
 def test_prompt_calls_captured_cold():
