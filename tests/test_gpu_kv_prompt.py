@@ -1,8 +1,9 @@
 """A prompt of more than 8 rows through the dense layer
 (kv_dense_layer_prefill_u16_ext_packed_rows8: all rows through each step
 together) against the oracle's one row at a time: token counts at the edges
-of the token tiles and of the 128-row passes, partial row tiles, K slices,
-heads of every kernel variant, over an earlier context with tentative rows.
+of the token tiles and of the 128-row passes, partial row tiles, 1 to 16 K
+slices, every token-tile count in both types, heads of every kernel variant,
+over an earlier context with tentative rows.
 
 Bar: rel-L2 1e-3 a row, that of the decode steps' test (the layer's 16-bit
 roundings, which a sum in another order can turn the other way).
@@ -37,6 +38,10 @@ def nat():
     (torch.bfloat16, True, (896, 1184, 14, 2), 200, 129),  # two passes
     (torch.float16, True, (1024, 256, 4, 1), 40, 20),    # heads of 256
     (torch.float16, False, (480, 256, 12, 4), 20, 12),   # heads of 40
+    (torch.bfloat16, False, (256, 5120, 4, 2), 10, 24),  # two token tiles, 16 K slices
+    (torch.float16, True, (512, 1056, 8, 8), 33, 40),    # four token tiles
+    (torch.float16, False, (256, 512, 4, 2), 0, 128),    # one whole pass
+    (torch.bfloat16, True, (480, 256, 12, 4), 20, 100),  # eight token tiles, one K slice
     (torch.float16, False, (288, 272, 9, 3), 20, 12),    # 272 columns: one row at a time
 ])
 def test_prompt_rows_match_the_oracle(nat, dtype, extras, shape, ctx, rows):
@@ -76,6 +81,68 @@ def test_prompt_rows_match_the_oracle(nat, dtype, extras, shape, ctx, rows):
         ours.dense_layer_prefill_packed_rows8(1, _t(hidden, dtype).reshape(rows, H), *dev_w, hidden_size=H,
                                               intermediate_size=I, **kw, **opt)
     ours.close()
+
+
+def _decoded(session, hidden, weights, **kw):
+    outs = []
+    for row in hidden:
+        outs.append(session.dense_layer_decode_packed_rows8(0, row, *weights, **kw))
+        session.commit(1)
+    return torch.stack(outs)
+
+
+def test_prompt_over_a_long_context_takes_several_attention_launches(nat):
+    """8300 earlier rows, 126 of the 128 prompt rows' partials in 64 MB: the
+    last two rows go in a launch of their own.  Rows against decode steps, the
+    bar of the tests above."""
+    H, I, nh, nkv, ctx, rows = 1024, 256, 16, 1, 8300, 130
+    w, norms, extra, rng = _layer(5, H, I, nh, nkv, 0, False, scale=0.02)
+    weights, opt = _device_layer(nat, w, norms, extra, torch.float16)
+    kw = dict(hidden_size=H, intermediate_size=I, num_heads=nh, num_kv_heads=nkv, rms_eps=1e-6, rope_theta=1e4, **opt)
+    kvw = H // nh * nkv
+    pre = [_t(kvo.f32_to_u16(rng.standard_normal((ctx, kvw)).astype(np.float32), 0), torch.float16) for _ in range(2)]
+    hidden = _t(kvo.f32_to_u16(rng.standard_normal((rows, H)).astype(np.float32), 0), torch.float16)
+    results = []
+    for run in (lambda s: s.dense_layer_prefill_packed_rows8(0, hidden, *weights, **kw),
+                lambda s: _decoded(s, hidden, weights, **kw)):
+        s = nat.NativeKvSession(layer_count=1, max_seq_len=ctx + rows, kv_width=kvw, dtype=torch.float16)
+        s.append_committed(0, *pre, count=ctx)
+        results.append([run(s).double(), *(t[ctx:].double() for t in s.copy_layer(0))])
+        s.close()
+    for a, b in zip(*results):
+        rel = (a - b).norm(dim=1) / b.norm(dim=1)
+        assert rel.max() <= 1e-3, rel.max()
+
+
+@pytest.mark.parametrize("dtype,cases", [(torch.float16, ("inf", "nan", "values")), (torch.bfloat16, ("inf", "nan"))])
+def test_infinities_and_nans_stay_in_their_rows(nat, dtype, cases):
+    """A hidden row with an infinity, one with a NaN (last, since later rows
+    see their keys) and value rows that overflow fp16 (bf16 has fp32's range:
+    there the sums overflow, in either order): NaN and infinity where decode
+    steps have them, the other rows as without."""
+    H, I, nh, nkv, rows = 256, 512, 8, 2, 24
+    dc = 1 if dtype == torch.bfloat16 else 0
+    w, norms, extra, rng = _layer(6, H, I, nh, nkv, dc, False, scale=0.02)
+    hidden = _t(kvo.f32_to_u16(rng.standard_normal((rows, H)).astype(np.float32), dc), dtype)
+    kw = dict(hidden_size=H, intermediate_size=I, num_heads=nh, num_kv_heads=nkv, rms_eps=1e-6, rope_theta=1e4)
+    for case in cases:
+        x = hidden.clone()
+        if case == "values":
+            w = dict(w, v=kvo.f32_to_u16((rng.standard_normal((nkv * H // nh, H)) * 4096).astype(np.float32), dc))
+        else:
+            x[rows - 1, 3] = float(case)
+        weights, opt = _device_layer(nat, w, norms, extra, dtype)
+        results = []
+        for run in (lambda s: s.dense_layer_prefill_packed_rows8(0, x, *weights, **kw, **opt),
+                    lambda s: _decoded(s, x, weights, **kw, **opt)):
+            s = nat.NativeKvSession(layer_count=1, max_seq_len=rows, kv_width=H // nh * nkv, dtype=dtype)
+            results.append([run(s), *s.copy_layer(0)])
+            s.close()
+        assert any(not torch.isfinite(t).all() for t in results[1]), case
+        for a, b in zip(*results):
+            assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf()), case
+            a, b = (t.nan_to_num(0.0, 0.0, 0.0).double() for t in (a, b))
+            assert ((a - b).norm(dim=1) <= 1e-3 * b.norm(dim=1)).all(), case
 
 
 def _cancelling_layer(nat, which, dtype, H, I, nh, nkv, perm):

@@ -100,9 +100,9 @@ def test_argument_errors(nat):
 @pytest.mark.parametrize("rows", [3, 64, 65, 1024, 1025, 9000])
 @pytest.mark.parametrize("levels", [1, 2, 40])
 def test_selection_among_few_distinct_logits(nat, rows, levels):
-    """Logits of 1, 2 or 40 distinct values (zeros and negative zeros among
-    them), so that the threshold search ends on ties, between them, or with
-    exactly top_k entries above it: the largest first, equal ones in row order."""
+    """Logits of 1, 2 or 40 distinct values (zero among them), so that the
+    threshold search ends on ties, between them, or with exactly top_k entries
+    above it: the largest first, equal ones in row order."""
     g = torch.Generator().manual_seed(rows + levels)
     value = (torch.randint(0, levels, (rows,), generator=g) - levels // 2).float() * 0.25
     weight = torch.zeros((rows, 8), dtype=torch.float16)
