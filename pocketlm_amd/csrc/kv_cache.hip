@@ -526,17 +526,17 @@ bool launch_split_g(int tok, int vd, dim3 grid, size_t lds, hipStream_t st, cons
                     float* part, float* ml) {
     if constexpr (G >= 4) {
         if (tok == 16)
-            return launch_split_t<BF16, G, 16, false>(vd, grid, lds, st, q_rot, kc, vc, kvw, hd, group, T, scale, vec, slots,
-                                               part, ml);
+            return launch_split_t<BF16, G, 16, false>(vd, grid, lds, st, q_rot, kc, vc, kvw, hd, group, T, scale, vec,
+                                                      slots, part, ml);
     }
     if constexpr (G >= 2) {
         if (tok == 32)
-            return launch_split_t<BF16, G, 32, false>(vd, grid, lds, st, q_rot, kc, vc, kvw, hd, group, T, scale, vec, slots,
-                                               part, ml);
+            return launch_split_t<BF16, G, 32, false>(vd, grid, lds, st, q_rot, kc, vc, kvw, hd, group, T, scale, vec,
+                                                      slots, part, ml);
     }
     if (tok != 64) return false;
-    return launch_split_t<BF16, G, 64, false>(vd, grid, lds, st, q_rot, kc, vc, kvw, hd, group, T, scale, vec, slots, part,
-                                       ml);
+    return launch_split_t<BF16, G, 64, false>(vd, grid, lds, st, q_rot, kc, vc, kvw, hd, group, T, scale, vec, slots,
+                                              part, ml);
 }
 
 // Heads per kv head rounded up to the kernels' G.
@@ -777,11 +777,11 @@ __global__ __launch_bounds__(kNormThreads) void post_attention_kernel(const uint
 // A prompt through the layer takes up to kRow8BatchRows rows at a time
 // through each step, so that every weight is read once for all of them
 // (120 rows one at a time: 120 times; 3584 / 18944 in fp16, 120 rows: 13.6 ->
-// 0.40 ms a call).  The projections run on the matrix
-// cores (row8_batch.hip) and leave sums per K slice, which the next kernel
-// adds; activations go to them as planes of 16-bit values in the order
-// row8.h describes.  The values that a row's step rounds to the
-// storage type are rounded the same here; sums run in another order.
+// 0.45 ms a call).  The projections run on the matrix cores (row8_batch.hip)
+// and leave sums per K slice, which the next kernel adds; activations go to
+// them as planes of 16-bit values in the order row8.h describes.  The values
+// that a row's step rounds to the storage type are rounded the same here; sums
+// run in another order, as close to 64 bits as the decode step's.
 
 constexpr int kRowThreads = 1024;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -1332,11 +1332,11 @@ int commit_rows(KvSession* s, int64_t count) {
 }
 
 // A prompt: every row through the layer, then committed.  Prompts of up to
-// kPromptDecodeRows rows go one row at a time, so that they have the bits of
-// decode steps (a verifier's draft; 3584 / 18944: 8 rows 954 us a call, 9
-// rows together 256, 64 rows 319, 120 rows 393);
-// longer ones kRow8BatchRows at a time where the shape suits
-// the row kernels (whole 32-column steps, 16-byte K pieces).
+// kPromptDecodeRows rows go one row at a time: callers and tests hold a short
+// prefill to the bits of decode steps, which is worth more there than the time
+// (3584 / 18944 in fp16: 8 rows 1000 us a call, 9 rows together 262, 64 rows
+// 329, 120 rows 449).  Longer ones go kRow8BatchRows at a time where the shape
+// suits the row kernels (whole 32-column steps, 16-byte K pieces).
 constexpr int64_t kPromptDecodeRows = 8;
 
 template <bool BF16>
