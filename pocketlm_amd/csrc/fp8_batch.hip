@@ -82,7 +82,7 @@ __global__ __launch_bounds__(64 * MAXW) void fp8_batch_kernel(const BatchArgs a)
     int64_t obase = a.base != nullptr ? a.base[g] : g * a.m;
     int64_t rows = a.rows;
     float* out = a.out;
-    if (!SILU && a.nouts > 0) {
+    if (!SILU && XM != kXPlanes && a.nouts > 0) {
         rows = a.out_rows[g];
         out = a.outs[g];
         obase = 0;
