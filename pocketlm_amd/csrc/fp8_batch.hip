@@ -15,9 +15,9 @@
 // a one-row call.
 //
 // Measured on an MI355X against passes of 8 rows: 7168x16384 at 16 bf16 rows
-// 52 -> 40 us, at 64 rows 226 -> 78 us; 96 rows of top-8 over 256 experts of
-// 7168/2048 27.2 -> 2.02 ms (5.3 TB/s: the weights of every chosen expert,
-// read once).
+// 61 -> 45 us, at 64 rows 212 -> 83 us, 2048x7168 at 9 and 16 rows 14.4 -> 11.4
+// and 16.1 -> 13.6; 96 rows of top-8 over 256 experts of 7168/2048 27.2 -> 2.02
+// ms (5.3 TB/s: the weights of every chosen expert, read once).
 #include <algorithm>
 #include <cstring>
 #include <type_traits>
@@ -434,11 +434,12 @@ __global__ __launch_bounds__(kPairThreads) void pair_sum_kernel(const float* __r
 // bits.
 //
 // What bounds it: a wave's own instructions (at one to two waves per SIMD
-// conversions, scaling FMAs, MFMAs and LDS reads hardly overlap; more
-// workgroups per compute unit, deeper prefetch or single buffers changed
-// nothing).  24576x1536 at 509 bf16 rows: 289 us with the skinny kernel, 75
-// here (510 TFLOP/s) and 5 for packing; the 7168 / 2048 MLP at 256 fp32 rows
-// 251 -> 107 us (gate + up 74, down 38).
+// conversions, scaling FMAs, MFMAs and LDS reads hardly overlap: of the busy
+// cycles of the bf16 linear below the vector units issue in 46 %, the matrix
+// cores and the LDS work in 25 % each; more workgroups per compute unit, deeper
+// prefetch or single buffers changed nothing).  24576x1536 at 509 bf16 rows:
+// 289 us with the skinny kernel, 75 here (510 TFLOP/s) and 5 for packing; the
+// 7168 / 2048 MLP at 256 fp32 rows 251 -> 107 us (gate + up 73, down 38).
 //
 // The activations come packed ([block][column tile][half][piece][lane]
 // [8 values], kTileBytes per column tile and block) by fp8_pack_rows_kernel,

@@ -28,7 +28,7 @@
 //
 // What bounds it: loads in flight and their spread.  At 120 rows of a 3584 /
 // 18944 layer in fp16 (us): q + k + v 27, o 29, gate + up 126 (2.2 TB/s),
-// down 115.  Sums kept in the matrix instruction and two fp16 parts took 27,
+// down 113.  Sums kept in the matrix instruction and two fp16 parts took 27,
 // 25, 112 and 94.  The whole layer 13.6 ms one row at a time -> 0.39 ms of
 // kernels.
 #include <algorithm>
